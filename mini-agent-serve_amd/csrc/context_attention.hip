@@ -130,12 +130,13 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
 
 // A raw buffer resource: no stride, `bytes` records (a load at a byte offset past them returns
 // zeros), dword 3 = 0x00020000 (the 32-bit data format that untyped buffer loads take on gfx9).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const uint16_t* base, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, bytes, 0x00020000);
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const char* base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, bytes, 0x00020000);
 }
 // LDS DMA: lane i of the wavefront writes the 16 bytes at byte offset voffset of resource r to LDS
 // address dst + 16 i (dst wavefront-uniform); zeros for an offset past the resource's records.
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, uint16_t* dst, int voffset) {
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, lds_u16* dst, int voffset) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(dst), 16, voffset, 0, 0, 0);
 }
 // s_waitcnt vmcnt(0) (expcnt and lgkmcnt fields at their maxima: not waited on)
@@ -693,7 +694,7 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   // start of the page for each k < MQ (the same for every page).
   constexpr int PS = kMulti ? (8 << (kPages - kPagesMulti8)) : kTileP;  // rows per page (kMulti)
   constexpr int PT = kTileP / PS;                                         // pages per tile
-  constexpr int PPW = (PT + kCtxWaves - 1) / kCtxWaves;                   // pages per wavefront, at most
+  constexpr int PPW = (PT + kCtxWaves - 1) / kCtxWaves;                   // pages per wavefront, at most (1: one-page tiles)
   constexpr int MQK = kMulti ? (PS * SK + 63) / 64 : NK, MQV = kMulti ? (PS * SV + 63) / 64 : NV;
   int koff[MQK], voff[MQV];
   if constexpr (kDirect) {
@@ -705,52 +706,74 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
 #pragma unroll
     for (int j = 0; j < MQV; ++j) voff[j] = place(64 * (kMulti ? j : wave + kCtxWaves * j) + lane, SV);
   }
-  struct TileRsrc {
-    __amdgpu_buffer_rsrc_t k, v;
-  };
-  // The block table through the constant address space: a scalar load (the DMA instructions would
-  // otherwise keep the compiler from proving the table unwritten, and it would load the page id
-  // with a vector load and wait on every load in flight).
+  // Page ids: lane i holds block-table entry 64 page_chunk + i (clamped to the sequence's last one),
+  // read back with readlane, so finding a tile's page costs no memory round trip. The next 64 entries
+  // load a tile before their first use, and the wait for the tiles' own DMA covers them. The first two
+  // tiles' ids are scalar loads (constant address space: the DMA instructions would otherwise keep the
+  // compiler from proving the table unwritten), which overlap the query loads. A tile's
+  // pages are found once, for its keys; its values, a step later, reuse the offsets. (Two scalar
+  // loads per step, each waited for after the step's barrier, and the address arithmetic of both
+  // tiles took 3% of the call: 1634 -> 1590 us at 4 x 4096 tokens of 96 heads over 8, 202 -> 196 us at 6
+  // ragged prompts of 32 heads.)
   const auto bt_const = (const __attribute__((address_space(4))) int32_t*)(bt);
-  auto tile_rsrc = [&](int base) {
-    const int32_t page = bt_const[base >> a.log2_page];
-    const bool ok = page >= 0 && page < a.num_pages;
-    page_bad |= !ok;
-    const int64_t off = (ok ? static_cast<int64_t>(page) : 0) * a.page_stride +
-                        static_cast<int64_t>(base & pmask) * a.entry_stride + kvh * a.head_stride;
-    const int bytes = ok ? static_cast<int>(min(kTileP, kv_len - base) * a.entry_stride) * 2 : 0;
-    return TileRsrc{make_rsrc(a.k_cache + off, bytes), make_rsrc(a.v_cache + off, bytes)};
+  int page_ids = 0, next_page_ids = 0, page_chunk = 0;
+  const uint32_t pages_u32 = static_cast<uint32_t>(min(a.num_pages, static_cast<int64_t>(INT32_MAX)));
+  const auto load_page_ids = [&](int chunk) { return bt[min(64 * chunk + lane, last_page)]; };
+  struct TilePages {   // this wavefront's pages of a tile: byte offset in the caches, and valid bytes
+    int64_t off[PPW];
+    int bytes[PPW];
   };
-  // kMulti: the resource of page q of the tile at `base` (pages start at multiples of their size,
-  // and tiles at multiples of 64): based at the page's first row of this kv head, its records ending
-  // after the page's last position below kv_len. A page wholly past kv_len has no records (its
-  // block-table entry, read clamped to the sequence's last one, is not used).
-  auto page_rsrc = [&](const uint16_t* cache, int base, int q) {
-    const int pos = base + q * PS;
-    // (readfirstlane: the clamp is selected as a vector med3, and a resource dword in a vector
-    // register would make the compiler loop over its distinct values)
-    const int rows = __builtin_amdgcn_readfirstlane(max(0, min(kv_len - pos, PS)));
-    const int32_t page = bt_const[min(pos >> a.log2_page, last_page)];
-    const bool ok = page >= 0 && page < a.num_pages;
-    page_bad |= rows > 0 && !ok;
-    const int64_t off = (ok ? static_cast<int64_t>(page) : 0) * a.page_stride + kvh * a.head_stride;
-    return make_rsrc(cache + off, ok ? static_cast<int>(rows * a.entry_stride) * 2 : 0);
+  const char* const k_head = reinterpret_cast<const char*>(a.k_cache + kvh * a.head_stride);
+  const char* const v_head = reinterpret_cast<const char*>(a.v_cache + kvh * a.head_stride);
+  const uint64_t page_bytes = static_cast<uint64_t>(a.page_stride) * 2;
+  const int entry_bytes = static_cast<int>(a.entry_stride) * 2;  // kDirect: a tile's rows fit 31 bits
+  // The pages of the tile at `base`: one-page tiles from the tile's first row, kMulti from the first
+  // row of each page (pages start at multiples of their size, tiles at multiples of 64), the valid
+  // bytes ending after the last position below kv_len. A page wholly past kv_len has none, nor has
+  // one whose id is outside the cache.
+  auto chunk_of = [&](int base) { return base >> a.log2_page >> 6; };
+  auto find_pages = [&](int base, bool prologue) {
+    if (!prologue) {
+      const int chunk = chunk_of(base), next = chunk_of(base + kTileP);
+      if (chunk != page_chunk) {  // uniform
+        page_ids = next_page_ids;
+        page_chunk = chunk;
+      }
+      if (next != chunk) next_page_ids = load_page_ids(next);
+    }
+    TilePages t;
+#pragma unroll
+    for (int pj = 0; pj < PPW; ++pj) {
+      const int pos = kMulti ? base + (wave + kCtxWaves * pj) * PS : base;
+      // (readfirstlane: the clamp is selected as a vector med3, and a resource dword in a vector
+      // register would make the compiler loop over its distinct values)
+      const int rows = __builtin_amdgcn_readfirstlane(max(0, min(kv_len - pos, PS)));
+      const int entry = pos >> a.log2_page;
+      const uint32_t page = static_cast<uint32_t>(prologue ? bt_const[min(entry, last_page)]
+                                                           : __builtin_amdgcn_readlane(page_ids, entry & 63));
+      const bool ok = page < pages_u32;
+      page_bad |= rows > 0 && !ok;
+      t.off[pj] = static_cast<int64_t>((ok ? page : 0u) * page_bytes);
+      if constexpr (!kMulti) t.off[pj] += static_cast<int64_t>(pos & pmask) * entry_bytes;
+      t.bytes[pj] = ok ? rows * entry_bytes : 0;
+    }
+    return t;
   };
   // One tile's keys or values into `dst`, this wavefront's instructions. The LDS addresses are
   // formed where the loads issue (the opaque copy of the buffer's address keeps the compiler from
   // hoisting twenty of them out of the tile loop into spilled registers).
-  auto dma_part = [&](bool keys, int base, uint16_t* dst) {
-    const uint16_t* cache = keys ? a.k_cache : a.v_cache;
-    uint16_t* d = dst;
+  auto dma_part = [&](bool keys, const TilePages& t, uint16_t* dst) {
+    const char* cache = keys ? k_head : v_head;
+    lds_u16* d = (lds_u16*)dst;
     asm volatile("" : "+s"(d));
     if constexpr (kMulti) {
 #pragma unroll
       for (int pj = 0; pj < PPW; ++pj) {
         const int q = wave + kCtxWaves * pj;
         if (q >= PT) continue;  // wavefront-uniform
-        const __amdgpu_buffer_rsrc_t r = page_rsrc(cache, base, q);
+        const __amdgpu_buffer_rsrc_t r = make_rsrc(cache + t.off[pj], t.bytes[pj]);
         const int S = keys ? SK : SV;
-        uint16_t* dq = d + 8 * q * PS * S;
+        lds_u16* dq = d + 8 * q * PS * S;
         constexpr int MQ = MQK > MQV ? MQK : MQV;
 #pragma unroll
         for (int k = 0; k < MQ; ++k) {
@@ -761,19 +784,19 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
         }
       }
     } else {
-      const TileRsrc t = tile_rsrc(base);
+      const __amdgpu_buffer_rsrc_t r = make_rsrc(cache + t.off[0], t.bytes[0]);
       constexpr int N = NK > NV ? NK : NV;
 #pragma unroll
       for (int j = 0; j < N; ++j) {
         if (keys ? j >= NK : j >= NV) continue;
         const int m = wave + kCtxWaves * j;
         if (m >= (keys ? SK : SV)) continue;
-        dma16(keys ? t.k : t.v, d + 512 * m, keys ? koff[j] : voff[j]);
+        dma16(r, d + 512 * m, keys ? koff[j] : voff[j]);
       }
     }
   };
-  auto dma_keys = [&](int base, uint16_t* dst) { dma_part(true, base, dst); };
-  auto dma_values = [&](int base, uint16_t* dst) { dma_part(false, base, dst); };
+  auto dma_keys = [&](const TilePages& t, uint16_t* dst) { dma_part(true, t, dst); };
+  auto dma_values = [&](const TilePages& t, uint16_t* dst) { dma_part(false, t, dst); };
 
   // kPagesLane: each lane reads the page of each of its rows; rows past kv_len load the sequence's
   // last row and are zeroed when staged, as are rows on a page id outside the cache (page 0 read).
@@ -940,11 +963,18 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   // step, after this wavefront's DMA of the previous step has landed, covers both: every wavefront's
   // loads are in LDS, and every read of the buffers refilled next is done.
   f32x16 s_a[2], s_b[2];
+  TilePages ahead{};  // kDirect: the pages of the tile whose keys the DMA took last
   if (it_begin < it_end) {
     if constexpr (kDirect) {
-      dma_keys(it_begin * kTileP, klds(0));
-      dma_values(it_begin * kTileP, vlds(0));
-      if (it_begin + 1 < it_end) dma_keys((it_begin + 1) * kTileP, klds(1));
+      ahead = find_pages(it_begin * kTileP, true);
+      dma_keys(ahead, klds(0));
+      dma_values(ahead, vlds(0));
+      if (it_begin + 1 < it_end) {
+        ahead = find_pages((it_begin + 1) * kTileP, true);
+        dma_keys(ahead, klds(1));
+      }
+      page_chunk = chunk_of((it_begin + 2) * kTileP);
+      page_ids = load_page_ids(page_chunk);
       __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
       __syncthreads();
     } else {
@@ -961,8 +991,11 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
     if constexpr (kDirect) {
       __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
       __syncthreads();
-      if (it + 1 < it_end) dma_values((it + 1) * kTileP, vlds(buf ^ 1));
-      if (it + 2 < it_end) dma_keys((it + 2) * kTileP, klds(buf));
+      if (it + 1 < it_end) dma_values(ahead, vlds(buf ^ 1));
+      if (it + 2 < it_end) {
+        ahead = find_pages((it + 2) * kTileP, false);
+        dma_keys(ahead, klds(buf));
+      }
     } else {
       __syncthreads();  // tile it - 1's reads (of buffer buf ^ 1) are done
       if (it + 1 < it_end) stage(tr, buf ^ 1);
