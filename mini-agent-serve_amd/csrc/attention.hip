@@ -136,12 +136,6 @@ constexpr int kAttnWaves = 1;
 // Wavefronts per SIMD the split kernel's registers are capped for (two load buffers of a step each).
 constexpr int kAttnMinWaves = 2;
 
-// Orders this wavefront's LDS writes before its later reads (and reads before later writes).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // One step: 32 positions - two MFMA tiles of keys, and the value rows in the 16-byte layout.
 template <int D>
 struct StepLoads {

@@ -22,10 +22,19 @@
 //   is read from the row-major value tile with gfx950's transposing LDS read (ds_read_b64_tr_b16:
 //   in each group of 16 lanes, lane 4a + b receives element b of the 4-element rows that lanes
 //   a, a + 4, a + 8, a + 12 point at), two per operand, in the position order the packing implies.
-// Tiles are software-pipelined over two LDS buffers each of keys and values: while tile i is in the
-// softmax, tile i + 1's score MFMAs run. With pages of at least a tile, the tiles go to LDS by DMA,
-// keys a tile ahead of values (tile i + 2's keys and tile i + 1's values in flight), one barrier
-// per tile; smaller pages stage tile i + 2 through registers, two barriers per tile.
+// A tile is worked through in two halves of 32 positions. One half's step runs three independent
+// parts side by side: the score MFMAs of the next half, the softmax weights of this one, and the P.V
+// MFMAs of the one before, so the matrix pipe and the vector ALU both have work that waits for nothing.
+// Keys and values have two LDS buffers each. With pages of at least 8 slots the tiles go to LDS by DMA,
+// issued among the MFMAs, keys a tile ahead of values (tile i + 2's keys and tile i + 1's values in
+// flight), one barrier per tile; smaller pages stage a tile through registers, two barriers per tile.
+// What bounds it: the card's power (the clock settles near 2 GHz under this load, and falls as the loop
+// gets denser), the 32 MFMAs per tile and wavefront (2048 of about 3200 cycles per tile for a SIMD's two
+// wavefronts), and the latency of the tiles' loads. Before the halves, the unpadded LDS rows (32 DMA
+// instructions per tile for 35 or 40, no bank conflicts) and the DMA among the MFMAs, a tile's scores
+// ran beside the whole previous tile's softmax, which waited for its maximum: 4 x 4096 tokens of 96 heads
+// over 8 took 1656 us, now 1571 (1050 TFLOP/s; a large bf16 matrix product reaches 1537 on this card);
+// 4 x 2048 of 32 heads 158 -> 150 us, 6 ragged prompts after cached ones 206 -> 191 us.
 #include <algorithm>
 
 #include "device.h"
@@ -37,8 +46,8 @@ constexpr int kTileP = 64;        // key positions per tile
 constexpr int kRowsPerWave = 32;  // query rows (tokens of one head) per wavefront
 constexpr int kMaxCtxSplits = 32;  // split-KV: key-range splits per token tile, at most
 constexpr float kNegInf = -__builtin_huge_valf();
-// The online softmax's lazy reference point: p = 2^(s c - m c) stays below 2^kLazyLog2.
-constexpr float kLazyLog2 = 8.f;
+// The online softmax's lazy reference point: a half tile's p = 2^(s c - m c) sum to at most this per lane.
+constexpr float kSumMost = 256.f;
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
@@ -511,17 +520,23 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   constexpr int kCtxThreads = 64 * kWaves;
   constexpr int KS = D / 16;            // MFMA k-steps over the head dim (S^T)
   constexpr int DB = D / 32;            // 32-dim blocks of O^T
-  constexpr int KROW = D + 8;           // bf16 per LDS key row (+16 B: conflict-free A reads)
-  constexpr int VROW = D + 16;          // bf16 per LDS value row (+32 B: conflict-free column reads)
   constexpr int CPR = D / 8;            // 16-byte chunks per key / value row
   constexpr int LOADS = kTileP * CPR / kCtxThreads;  // 16-byte chunks per thread per tile, each of K and V
   // Two tile buffers each of keys and values: with the software pipeline, the next tile's keys are
   // read while this tile's values are. Four separate arrays, so that the compiler's wait insertion
   // tells a buffer that an LDS DMA load is filling from the ones being read.
-  __shared__ __align__(16) uint16_t k_lds0[kTileP * KROW];
-  __shared__ __align__(16) uint16_t k_lds1[kTileP * KROW];
-  __shared__ __align__(16) uint16_t v_lds0[kTileP * VROW];
-  __shared__ __align__(16) uint16_t v_lds1[kTileP * VROW];
+  // Rows are D elements with no padding; a row's 16-byte chunk c sits in slot c ^ key_swizzle(row)
+  // (value_swizzle(row)), which spreads the rows of a key read and of a transposing value read over
+  // the banks.
+  __shared__ __align__(16) uint16_t k_lds0[kTileP * D];
+  __shared__ __align__(16) uint16_t k_lds1[kTileP * D];
+  __shared__ __align__(16) uint16_t v_lds0[kTileP * D];
+  __shared__ __align__(16) uint16_t v_lds1[kTileP * D];
+  // Rows in the same 16-byte column of the banks lie 16 / CPR rows apart. Keys: a 16-lane group reads
+  // one chunk of 16 consecutive rows. Values: 16 lanes read 32 bytes of each of 4 rows, the next 16
+  // lanes the next 32 bytes, the other half of the wavefront the same of the next 4 rows.
+  const auto key_swizzle = [](int row) { return (row / (16 / CPR)) & (CPR - 1); };
+  const auto value_swizzle = [](int row) { return (((row / (16 / CPR)) & (CPR / 4 - 1)) << 2) | (((row >> 2) & 1) << 1); };
   const auto klds = [&](int b) { return b ? k_lds1 : k_lds0; };
   const auto vlds = [&](int b) { return b ? v_lds1 : v_lds0; };
 
@@ -667,44 +682,33 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   struct TileRegs {
     u32x4 k[LOADS], v[LOADS];
     bool lok[LOADS];
-    bool full;  // every chunk of the tile valid: stores need no zeroing
   };
   bool page_bad = false;  // a real position's page id outside the cache (reported once, at the end)
   const int last_page = kv_len > 0 ? (kv_len - 1) >> a.log2_page : 0;  // the sequence's last block-table entry
 
   // ---- Pages of at least 8 slots (kDirect): the tiles go to LDS by DMA (buffer_load ... lds), with
   // no registers or stores in between. A wavefront's load instruction fills 64 consecutive 16-byte
-  // slots of an LDS tile buffer, lane i slot i. The buffers keep their row padding (SK / SV slots per
-  // key / value row, the last one or two of them padding), so lane i of an instruction that starts
-  // at a row's first slot loads row i / S, head-dim chunk i % S of the rows from there (a padding
-  // slot loads the row's last chunk once more). The rows are read through a buffer resource based at
-  // the first row of the tile (one-page tiles) or of the page (kMulti) of this kv head, its records
-  // ending after the last position below kv_len (none for a page id outside the cache): the rows past
-  // them arrive as zeros. The host keeps this mode to layouts whose in-page byte offsets fit 31 bits.
+  // slots of an LDS tile buffer, lane i slot i: RPI rows, lane i the chunk that its slot holds. The
+  // tile's rows are dealt out in order, NI instructions to each wavefront. They are read through a
+  // buffer resource based at the first row of the tile (one-page tiles) or of the page (kMulti) of
+  // this kv head, its records ending after the last position below kv_len (none for a page id outside
+  // the cache): the rows past them arrive as zeros. A wavefront's rows lie in PPW pages. The host
+  // keeps this mode to layouts whose in-page byte offsets fit 31 bits.
   constexpr bool kMulti = kPages >= kPagesMulti8;
   constexpr bool kDirect = kPages == kPagesTile || kMulti;
-  constexpr int SK = KROW / 8, SV = VROW / 8;  // 16-byte slots per LDS key / value row
-  constexpr int NK = (SK + kCtxWaves - 1) / kCtxWaves, NV = (SV + kCtxWaves - 1) / kCtxWaves;
-  // One-page tiles: instruction ii fills slots 64 ii .. 64 ii + 63 of the buffer, ii = wave + W j for
-  // this wavefront's j, and each lane keeps the byte offset of its row and chunk from the tile's
-  // first row.
-  // kMulti: page q of the tile (PS rows) fills the buffer's slots from q PS S on, in MQ = ceil(PS S /
-  // 64) instructions 64 slots apart (the last one with only the lanes inside the page's region).
-  // Page q is wavefront q % W's, and each lane keeps the byte offset of its row and chunk from the
-  // start of the page for each k < MQ (the same for every page).
   constexpr int PS = kMulti ? (8 << (kPages - kPagesMulti8)) : kTileP;  // rows per page (kMulti)
-  constexpr int PT = kTileP / PS;                                         // pages per tile
-  constexpr int PPW = (PT + kCtxWaves - 1) / kCtxWaves;                   // pages per wavefront, at most (1: one-page tiles)
-  constexpr int MQK = kMulti ? (PS * SK + 63) / 64 : NK, MQV = kMulti ? (PS * SV + 63) / 64 : NV;
-  int koff[MQK], voff[MQV];
+  constexpr int RPI = 64 / CPR, NI = kTileP / RPI / kCtxWaves;
+  constexpr int PPW = NI * RPI > PS ? NI * RPI / PS : 1;
+  const int my_row = wave * NI * RPI;  // this wavefront's first row of a tile
+  int koff[NI], voff[NI];
   if constexpr (kDirect) {
-    auto place = [&](int s, int S) {
-      return static_cast<int>((s / S) * a.entry_stride) * 2 + 16 * min(s % S, CPR - 1);
-    };
 #pragma unroll
-    for (int j = 0; j < MQK; ++j) koff[j] = place(64 * (kMulti ? j : wave + kCtxWaves * j) + lane, SK);
-#pragma unroll
-    for (int j = 0; j < MQV; ++j) voff[j] = place(64 * (kMulti ? j : wave + kCtxWaves * j) + lane, SV);
+    for (int j = 0; j < NI; ++j) {
+      const int r = my_row + j * RPI + lane / CPR;
+      const int at = (r % PS) * static_cast<int>(a.entry_stride) * 2;
+      koff[j] = at + 16 * ((lane % CPR) ^ key_swizzle(r));
+      voff[j] = at + 16 * ((lane % CPR) ^ value_swizzle(r));
+    }
   }
   // Page ids: lane i holds block-table entry 64 page_chunk + i (clamped to the sequence's last one),
   // read back with readlane, so finding a tile's page costs no memory round trip. The next 64 entries
@@ -732,7 +736,7 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   // bytes ending after the last position below kv_len. A page wholly past kv_len has none, nor has
   // one whose id is outside the cache.
   auto chunk_of = [&](int base) { return base >> a.log2_page >> 6; };
-  auto find_pages = [&](int base, bool prologue) {
+  auto find_pages = [&](int base, bool prologue, int limit) {
     if (!prologue) {
       const int chunk = chunk_of(base), next = chunk_of(base + kTileP);
       if (chunk != page_chunk) {  // uniform
@@ -744,10 +748,10 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
     TilePages t;
 #pragma unroll
     for (int pj = 0; pj < PPW; ++pj) {
-      const int pos = kMulti ? base + (wave + kCtxWaves * pj) * PS : base;
+      const int pos = kMulti ? base + (my_row / PS + pj) * PS : base;
       // (readfirstlane: the clamp is selected as a vector med3, and a resource dword in a vector
       // register would make the compiler loop over its distinct values)
-      const int rows = __builtin_amdgcn_readfirstlane(max(0, min(kv_len - pos, PS)));
+      const int rows = __builtin_amdgcn_readfirstlane(max(0, min(limit - pos, PS)));
       const int entry = pos >> a.log2_page;
       const uint32_t page = static_cast<uint32_t>(prologue ? bt_const[min(entry, last_page)]
                                                            : __builtin_amdgcn_readlane(page_ids, entry & 63));
@@ -759,49 +763,27 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
     }
     return t;
   };
-  // One tile's keys or values into `dst`, this wavefront's instructions. The LDS addresses are
-  // formed where the loads issue (the opaque copy of the buffer's address keeps the compiler from
-  // hoisting twenty of them out of the tile loop into spilled registers).
-  auto dma_part = [&](bool keys, const TilePages& t, uint16_t* dst) {
-    const char* cache = keys ? k_head : v_head;
-    lds_u16* d = (lds_u16*)dst;
-    asm volatile("" : "+s"(d));
-    if constexpr (kMulti) {
-#pragma unroll
-      for (int pj = 0; pj < PPW; ++pj) {
-        const int q = wave + kCtxWaves * pj;
-        if (q >= PT) continue;  // wavefront-uniform
-        const __amdgpu_buffer_rsrc_t r = make_rsrc(cache + t.off[pj], t.bytes[pj]);
-        const int S = keys ? SK : SV;
-        lds_u16* dq = d + 8 * q * PS * S;
-        constexpr int MQ = MQK > MQV ? MQK : MQV;
-#pragma unroll
-        for (int k = 0; k < MQ; ++k) {
-          if (k >= (keys ? MQK : MQV)) continue;
-          const int nact = min(64, PS * S - 64 * k);  // a constant
-          const int off = keys ? koff[k] : voff[k];
-          if (nact == 64 || lane < nact) dma16(r, dq + 512 * k, off);
-        }
-      }
-    } else {
-      const __amdgpu_buffer_rsrc_t r = make_rsrc(cache + t.off[0], t.bytes[0]);
-      constexpr int N = NK > NV ? NK : NV;
-#pragma unroll
-      for (int j = 0; j < N; ++j) {
-        if (keys ? j >= NK : j >= NV) continue;
-        const int m = wave + kCtxWaves * j;
-        if (m >= (keys ? SK : SV)) continue;
-        dma16(r, d + 512 * m, keys ? koff[j] : voff[j]);
-      }
-    }
+  // Instruction j of this wavefront's share of a tile's keys / values, into `dst`.
+  auto dma_key = [&](const TilePages& t, uint16_t* dst, int j) {
+    const int pj = j * PPW / NI;
+    dma16(make_rsrc(k_head + t.off[pj], t.bytes[pj]), (lds_u16*)dst + 64 * 8 * (wave * NI + j), koff[j]);
   };
-  auto dma_keys = [&](const TilePages& t, uint16_t* dst) { dma_part(true, t, dst); };
-  auto dma_values = [&](const TilePages& t, uint16_t* dst) { dma_part(false, t, dst); };
+  auto dma_value = [&](const TilePages& t, uint16_t* dst, int j) {
+    const int pj = j * PPW / NI;
+    dma16(make_rsrc(v_head + t.off[pj], t.bytes[pj]), (lds_u16*)dst + 64 * 8 * (wave * NI + j), voff[j]);
+  };
+  auto dma_keys = [&](const TilePages& t, uint16_t* dst) {
+#pragma unroll
+    for (int j = 0; j < NI; ++j) dma_key(t, dst, j);
+  };
+  auto dma_values = [&](const TilePages& t, uint16_t* dst) {
+#pragma unroll
+    for (int j = 0; j < NI; ++j) dma_value(t, dst, j);
+  };
 
   // kPagesLane: each lane reads the page of each of its rows; rows past kv_len load the sequence's
   // last row and are zeroed when staged, as are rows on a page id outside the cache (page 0 read).
   auto issue_tile = [&](TileRegs& tr, int base) {
-    tr.full = false;
 #pragma unroll
     for (int u = 0; u < LOADS; ++u) {
       const int p = base + prow + kPosStep * u;
@@ -820,134 +802,111 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   auto stage = [&](const TileRegs& tr, int buf) {
     uint16_t* k_lds = klds(buf);
     uint16_t* v_lds = vlds(buf);
-    if (tr.full) {
 #pragma unroll
-      for (int u = 0; u < LOADS; ++u) {
-        const int p = prow + kPosStep * u;
-        *reinterpret_cast<u32x4*>(k_lds + p * KROW + 8 * dcol) = tr.k[u];
-        *reinterpret_cast<u32x4*>(v_lds + p * VROW + 8 * dcol) = tr.v[u];
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < LOADS; ++u) {
-        const int p = prow + kPosStep * u;
-        const u32x4 kv = tr.lok[u] ? tr.k[u] : u32x4{0u, 0u, 0u, 0u};
-        const u32x4 vv = tr.lok[u] ? tr.v[u] : u32x4{0u, 0u, 0u, 0u};
-        *reinterpret_cast<u32x4*>(k_lds + p * KROW + 8 * dcol) = kv;
-        *reinterpret_cast<u32x4*>(v_lds + p * VROW + 8 * dcol) = vv;
-      }
+    for (int u = 0; u < LOADS; ++u) {
+      const int p = prow + kPosStep * u;
+      const u32x4 kv = tr.lok[u] ? tr.k[u] : u32x4{0u, 0u, 0u, 0u};
+      const u32x4 vv = tr.lok[u] ? tr.v[u] : u32x4{0u, 0u, 0u, 0u};
+      *reinterpret_cast<u32x4*>(k_lds + p * D + 8 * (dcol ^ key_swizzle(p))) = kv;
+      *reinterpret_cast<u32x4*>(v_lds + p * D + 8 * (dcol ^ value_swizzle(p))) = vv;
     }
   };
 
-  // Transposing-read coordinates of this lane's 16-lane group: head-dim column offset and row half.
-  const int grp_col = 16 * ((lane >> 4) & 1), k16 = lane & 15;
+  // This lane's offsets in a key half (k-step ks) and in 8 value rows (32-dim block db): the
+  // transposing read takes 4 columns of row 4 hf + k16 / 4 from it, in each 16-lane group columns
+  // 16 ((lane >> 4) & 1) + 4 (k16 % 4) .. + 3 of the block. (ks and db are bits apart from the rest: an
+  // exclusive or.)
+  const int k16 = lane & 15, v_row = 4 * hf + (k16 >> 2);
+  const int key_at0 = n * D + 8 * (hf ^ key_swizzle(n));
+  const int value_at0 = v_row * D + 8 * ((2 * ((lane >> 4) & 1) + ((k16 & 3) >> 1)) ^ value_swizzle(v_row)) + 4 * (k16 & 1);
   const float c = a.scale_log2;
-  // ---- S^T = K Q^T: element j of s[pb] holds S[token n][position base + 32 pb + 8 (j/4) + 4 hf + j%4]
-  auto scores = [&](int buf, f32x16 (&s)[2]) {
-    const uint16_t* k_lds = klds(buf);
-    bf16x8 ka[KS][2];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int pb = 0; pb < 2; ++pb)
-        ka[ks][pb] = *reinterpret_cast<const bf16x8*>(k_lds + (32 * pb + n) * KROW + 16 * ks + 8 * hf);
-    s[0] = f32x16{};
-    s[1] = f32x16{};
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int pb = 0; pb < 2; ++pb) s[pb] = mfma32(ka[ks][pb], qb[ks], s[pb]);
-    // the key reads run four ahead of the MFMAs that take them (the compiler's own order kept two in
-    // flight; eight ahead spills): 4 reads, then (MFMA, read) pairs, then the last 4 MFMAs
-    constexpr int kAhead = 4;
-    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);  // DS reads
-#pragma unroll
-    for (int i = 0; i < 2 * KS - kAhead; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // an MFMA
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // a DS read
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
+  // A tile is worked through in two halves of 32 positions. Half h = 2 i + b of tile i:
+  //   scores - S^T = K Q^T: element j of s holds S[token n][position base + 8 (j/4) + 4 hf + j%4];
+  //   weigh  - p = 2^(s c - m c), packed to bf16 as the B operands of O^T += V^T P^T: k-step kk =
+  //            positions 16 kk .. 16 kk + 15, lane half hf holding 16 kk + 4 hf + e (e < 4) and
+  //            16 kk + 8 + 4 hf + e - 4 (e >= 4), i.e. elements 8 kk .. + 7 of s;
+  //   pv     - O^T += V^T P^T: A = V^T[32 dims][16 positions], read transposed from the row-major
+  //            value tile in that position order.
+  auto key_op = [&](int buf, int half, int ks) {
+    return *reinterpret_cast<const bf16x8*>(klds(buf) + 32 * half * D + (key_at0 ^ 16 * ks));
   };
-  // ---- causal mask, only on tiles that cross the diagonal of the wavefront's first row or the end
+  auto value_op = [&](int buf, int kk, int db) {
+    const uint16_t* p = vlds(buf) + 16 * kk * D + (value_at0 ^ 32 * db);
+    const i16x4 lo = read_transposed4(p), hi = read_transposed4(p + 8 * D);
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  auto weigh = [&](const f32x16& s, float mc, bf16x8 (&pbo)[2]) {
+    float sum = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      float p[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * kk + e], c, -mc));
+        sum += p[e];
+      }
+      const u32x4 packed = {pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
+                            pack_bf16x2(p[6], p[7])};
+      pbo[kk] = __builtin_bit_cast(bf16x8, packed);
+    }
+    return sum;  // this lane's share: half of the row's 32
+  };
+  // ---- causal mask, only on halves that cross the diagonal of the wavefront's first row or the end
   // of the sequence (a wavefront-uniform branch)
-  auto mask = [&](f32x16 (&s)[2], int base) {
-    if (base + kTileP - 1 > shift + tok || base + kTileP > kv_len) {
-      // position kp is masked past min(this lane's query position, kv_len - 1); element j of s[pb]
-      // sits at kp = base + 4 hf + (32 pb + 8 (j / 4) + j % 4), the bracket a constant
+  auto mask = [&](f32x16& s, int base) {
+    if (base + 31 > shift + tok || base + 32 > kv_len) {
+      // position kp is masked past min(this lane's query position, kv_len - 1); element j of s sits at
+      // kp = base + 4 hf + (8 (j / 4) + j % 4), the bracket a constant
       const int lim = min(shift + tok + n, kv_len - 1) - base - 4 * hf;
 #pragma unroll
-      for (int pb = 0; pb < 2; ++pb)
-#pragma unroll
-        for (int j = 0; j < 16; ++j)
-          if (32 * pb + 8 * (j >> 2) + (j & 3) > lim) s[pb][j] = kNegInf;
+      for (int j = 0; j < 16; ++j)
+        if (8 * (j >> 2) + (j & 3) > lim) s[j] = kNegInf;
     }
   };
   // ---- online softmax per query row; scores stay in raw units, the scale enters the exponent
-  // through one fma: p = 2^(s c - m c). The reference point m is lazy: a row moves it only to a max
-  // more than kLazyLog2 above it (in exponent units), so p stays below 2^kLazyLog2 and O and l are
-  // rescaled (64 multiplies per lane) only when some row of the wavefront moved from a finite m;
-  // otherwise the stale m holds. bf16 P and the fp32 sums carry the same relative precision at any
-  // such magnitude, and O / l does not depend on m. The split partials carry this m with their sums.
-  // A row's 64 scores of a tile sit in lanes n and n + 32 (32 each). Whether any row must move its m
-  // is decided from each lane's own half (max(a, b) c exceeds a bound iff a c or b c does, c > 0), so
-  // the two halves exchange their maxima only on the seldom path that moves some m; each lane keeps
-  // its half's sum in l_run, and the halves are added once, after the last tile.
-  // P^T is packed to bf16 as the B operands of O^T += V^T P^T: k-step kk = positions 16 kk ..
-  // 16 kk + 15, lane half hf holding 16 kk + 4 hf + e (e < 4) and 16 kk + 8 + 4 hf + e - 4 (e >= 4),
-  // i.e. elements 8 (kk % 2) .. + 7 of s[kk / 2].
-  auto softmax = [&](f32x16 (&s)[2], bf16x8 (&pbo)[4]) {
-    float mh = kNegInf;  // this lane's half of the row
+  // through one fma. The reference point m is lazy: a half's p are taken against the m its row has,
+  // and only where a lane's 16 p sum to more than kSumMost does the wavefront move its rows' m to the
+  // maximum of their scores, rescale O and l, and take the half's p again. p stays below kSumMost, and
+  // bf16 P and the fp32 sums carry the same relative precision at any such magnitude; O / l does not
+  // depend on m. A row's first scores find m = -inf: their p are +inf (NaN for a masked score), which
+  // the test catches as well. The split partials carry this m with their sums. Each lane keeps its
+  // share of the sum in l_run; the two lanes of a row add theirs after the last tile.
+  auto move_reference = [&](const f32x16& s, bf16x8 (&pbo)[2]) {
+    float mh = kNegInf;
 #pragma unroll
-    for (int pb = 0; pb < 2; ++pb)
+    for (int j = 0; j < 16; ++j) mh = fmaxf(mh, s[j]);
+    const float m_new = fmaxf(m_run, fmaxf(mh, __shfl_xor(mh, 32)));  // the same in both lanes
+    // rows that had no finite score have O = 0 and l = 0: their factor is 1
+    const float alpha = m_run != kNegInf ? __builtin_amdgcn_exp2f(__builtin_fmaf(m_run, c, -(m_new * c))) : 1.f;
+    m_run = m_new;
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+      l_run *= alpha;
 #pragma unroll
-      for (int j = 0; j < 16; ++j) mh = fmaxf(mh, s[pb][j]);
-    // a row's first finite score (m = -inf) always moves it; -inf against -inf does not
-    const float bound = m_run * c + kLazyLog2;
-    if (__builtin_amdgcn_ballot_w64(mh * c > bound) != 0) {  // wavefront-uniform
-      const float mx = fmaxf(mh, __shfl_xor(mh, 32));        // the row's max, the same in both halves
-      const bool grow = mx * c > bound;
-      // rows that had no finite score have O = 0 and l = 0: their factor is 1
-      const float alpha = grow && m_run != kNegInf ? __builtin_amdgcn_exp2f(__builtin_fmaf(m_run, c, -(mx * c))) : 1.f;
-      if (grow) m_run = mx;
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
-        l_run *= alpha;
-#pragma unroll
-        for (int db = 0; db < DB; ++db) acc[db] *= alpha;
-      }
+      for (int db = 0; db < DB; ++db) acc[db] *= alpha;
     }
-    const float mc = (m_run == kNegInf ? 0.f : m_run) * c;
-    float sum = 0.f;
-#pragma unroll
-    for (int pb = 0; pb < 2; ++pb)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        s[pb][j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[pb][j], c, -mc));
-        sum += s[pb][j];
-      }
-    l_run += sum;  // this half's share
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const int o = 8 * (kk & 1);
-      const f32x16& sv = s[kk >> 1];
-      const u32x4 packed = {pack_bf16x2(sv[o], sv[o + 1]), pack_bf16x2(sv[o + 2], sv[o + 3]),
-                            pack_bf16x2(sv[o + 4], sv[o + 5]), pack_bf16x2(sv[o + 6], sv[o + 7])};
-      pbo[kk] = __builtin_bit_cast(bf16x8, packed);
-    }
+    return weigh(s, (m_run == kNegInf ? 0.f : m_run) * c, pbo);
   };
-  // ---- O^T += V^T P^T: A = V^T[32 dims][16 positions], read transposed from the row-major value
-  // tile in the position order of pbo
-  auto pv = [&](int buf, const bf16x8 (&pbo)[4]) {
-    const uint16_t* v_lds = vlds(buf);
+  auto settle = [&](float sum, const f32x16& s, bf16x8 (&pbo)[2]) {
+    if (__builtin_amdgcn_ballot_w64(!(sum <= kSumMost)) != 0) sum = move_reference(s, pbo);  // wavefront-uniform
+    l_run += sum;
+  };
+  // One half's work, the three parts of three different halves, so that none waits for another: the
+  // scores of half h + 1 (key half `khalf` of buffer kbuf) into `nxt`, the weights of half h (`cur`,
+  // masked) into pb_cur, and P.V of half h - 1 (value half `vhalf` of buffer vbuf). The score and P.V
+  // MFMAs alternate (a half's scores are one chain over the head dim), with the reads of the operands
+  // ahead of them and the weights' instructions between them.
+  auto half_step = [&](int kbuf, int khalf, f32x16& nxt, int vbuf, int vhalf, const bf16x8 (&pb_prev)[2],
+                       const f32x16& cur, bf16x8 (&pb_cur)[2], auto&& load) {
+    f32x16 sn{};
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-#pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        const i16x4 lo = read_column4(v_lds, VROW, 16 * kk + 4 * hf, 32 * db + grp_col, k16);
-        const i16x4 hi = read_column4(v_lds, VROW, 16 * kk + 8 + 4 * hf, 32 * db + grp_col, k16);
-        const bf16x8 va = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        acc[db] = mfma32(va, pbo[kk], acc[db]);
-      }
+    for (int i = 0; i < KS; ++i) {
+      sn = mfma32(key_op(kbuf, khalf, i), qb[i], sn);
+      acc[i % DB] = mfma32(value_op(vbuf, 2 * vhalf + i / DB, i % DB), pb_prev[i / DB], acc[i % DB]);
+      load(i);
     }
+    const float sum = weigh(cur, m_run * c, pb_cur);
+    nxt = sn;
+    settle(sum, cur, pb_cur);
   };
 
   TileRegs tr;
@@ -962,15 +921,16 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   // tile it + 2 and value buffer buf ^ 1 (tile it - 1's values) with tile it + 1. One barrier per
   // step, after this wavefront's DMA of the previous step has landed, covers both: every wavefront's
   // loads are in LDS, and every read of the buffers refilled next is done.
-  f32x16 s_a[2], s_b[2];
+  f32x16 s_even{}, s_odd{};   // the scores of a tile's halves
+  bf16x8 pb_even[2], pb_odd[2];  // and their weights
   TilePages ahead{};  // kDirect: the pages of the tile whose keys the DMA took last
   if (it_begin < it_end) {
     if constexpr (kDirect) {
-      ahead = find_pages(it_begin * kTileP, true);
+      ahead = find_pages(it_begin * kTileP, true, kv_len);
       dma_keys(ahead, klds(0));
       dma_values(ahead, vlds(0));
       if (it_begin + 1 < it_end) {
-        ahead = find_pages((it_begin + 1) * kTileP, true);
+        ahead = find_pages((it_begin + 1) * kTileP, true, kv_len);
         dma_keys(ahead, klds(1));
       }
       page_chunk = chunk_of((it_begin + 2) * kTileP);
@@ -983,39 +943,79 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
       __syncthreads();
       if (it_begin + 1 < it_end) issue_tile(tr, (it_begin + 1) * kTileP);
     }
-    if (wave_live) scores(0, s_a);
+    if (wave_live) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        s_even = mfma32(key_op(0, 0, ks), qb[ks], s_even);
+        s_odd = mfma32(key_op(0, 1, ks), qb[ks], s_odd);
+      }
+      mask(s_even, it_begin * kTileP);
+      l_run = move_reference(s_even, pb_even);
+    }
   }
-  // One tile in buffer `buf`; `cur` holds its scores, `nxt` receives the next tile's. Called with
-  // the two score arrays in turn (no copy between them).
-  auto step = [&](int it, int buf, f32x16 (&cur)[2], f32x16 (&nxt)[2]) {
+  // One tile in value buffer `buf`: its second half's weights and both halves' P.V, and the next tile's
+  // scores and its first half's weights.
+  auto step = [&](int it, int buf) {
+    TilePages value_pages{};
     if constexpr (kDirect) {
       __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
       __syncthreads();
-      if (it + 1 < it_end) dma_values(ahead, vlds(buf ^ 1));
-      if (it + 2 < it_end) {
-        ahead = find_pages((it + 2) * kTileP, false);
-        dma_keys(ahead, klds(buf));
-      }
+      value_pages = ahead;
+      ahead = find_pages((it + 2) * kTileP, false, it + 2 < it_end ? kv_len : 0);
     } else {
       __syncthreads();  // tile it - 1's reads (of buffer buf ^ 1) are done
-      if (it + 1 < it_end) stage(tr, buf ^ 1);
+      stage(tr, buf ^ 1);
       __syncthreads();
       if (it + 2 < it_end) issue_tile(tr, (it + 2) * kTileP);
     }
+    auto load_value = [&](int j) {
+      if constexpr (kDirect) {
+        if (j < NI) dma_value(value_pages, vlds(buf ^ 1), j);
+      }
+    };
+    auto load_key = [&](int j) {
+      if constexpr (kDirect) {
+        if (j < NI) dma_key(ahead, klds(buf), j);
+      }
+    };
     if (wave_live) {
-      mask(cur, it * kTileP);
-      bf16x8 pbo[4];
-      scores(buf ^ 1, nxt);  // the next tile's (stale buffer contents after the last tile: unused)
-      softmax(cur, pbo);
-      pv(buf, pbo);
+      mask(s_odd, it * kTileP + 32);
+      half_step(buf ^ 1, 0, s_even, buf, 0, pb_even, s_odd, pb_odd, load_value);
+      mask(s_even, (it + 1) * kTileP);
+      half_step(buf ^ 1, 1, s_odd, buf, 1, pb_odd, s_even, pb_even, load_key);
+    } else if constexpr (kDirect) {
+      dma_values(value_pages, vlds(buf ^ 1));
+      dma_keys(ahead, klds(buf));
+    }
+  };
+  auto last_step = [&](int it, int buf) {
+    if constexpr (kDirect) __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+    __syncthreads();
+    if (wave_live) {
+      auto pv = [&](int half, const bf16x8 (&pb)[2]) {
+#pragma unroll
+        for (int i = 0; i < KS; ++i) acc[i % DB] = mfma32(value_op(buf, 2 * half + i / DB, i % DB), pb[i / DB], acc[i % DB]);
+      };
+      mask(s_odd, it * kTileP + 32);
+      pv(0, pb_even);
+      if (it * kTileP + 32 <= shift + tok + kRowsPerWave - 1) {  // else no row sees the second half
+        const float sum = weigh(s_odd, m_run * c, pb_odd);
+        settle(sum, s_odd, pb_odd);
+        pv(1, pb_odd);
+      }
     }
   };
   int it = it_begin;
-  for (; it + 1 < it_end; it += 2) {
-    step(it, 0, s_a, s_b);
-    step(it + 1, 1, s_b, s_a);
+  for (; it + 2 < it_end; it += 2) {
+    step(it, 0);
+    step(it + 1, 1);
   }
-  if (it < it_end) step(it, 0, s_a, s_b);
+  if (it + 1 < it_end) {
+    step(it, 0);
+    last_step(it + 1, 1);
+  } else if (it < it_end) {
+    last_step(it, 0);
+  }
   if (__builtin_amdgcn_ballot_w64(page_bad) != 0 && lane == 0) report(a.err, MAS_ERRBIT_PAGE);
   // reported by the workgroup of token tile 0, which every row with a query token has
   if (len_bad && tid == 0 && blockIdx.x == 0 && tile_idx == 0) report(a.err, MAS_ERRBIT_POSITION);

@@ -160,13 +160,21 @@ __device__ __forceinline__ float block_sum(float v, float* slots) {
          (((a2[0] + a2[1]) + (a2[2] + a2[3])) + ((a3[0] + a3[1]) + (a3[2] + a3[3])));
 }
 
+// Orders this wavefront's LDS writes before its later reads (and reads before later writes).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Four values of one column of a row-major bf16 tile in LDS (rows vrow elements apart) from four
 // consecutive rows, with gfx950's transposing LDS read: in each group of 16 lanes, lane k points
 // at row first + k / 4, columns col0 + 4 (k % 4) .. + 3; lane n then holds rows first .. first + 3
 // of column col0 + n.
-__device__ __forceinline__ i16x4 read_column4(const uint16_t* lds_tile, int vrow, int first, int col0, int k) {
-  const uint16_t* p = lds_tile + (first + (k >> 2)) * vrow + col0 + 4 * (k & 3);
+__device__ __forceinline__ i16x4 read_transposed4(const uint16_t* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)(p));
+}
+__device__ __forceinline__ i16x4 read_column4(const uint16_t* lds_tile, int vrow, int first, int col0, int k) {
+  return read_transposed4(lds_tile + (first + (k >> 2)) * vrow + col0 + 4 * (k & 3));
 }
 
 __device__ __forceinline__ void report(uint32_t* err, uint32_t bit) {

@@ -1,0 +1,53 @@
+"""Context attention's 32-position half steps at their edges, against the oracle: lengths around whole
+halves and tiles, for every workgroup shape and page mode, with scores whose running reference has to
+move in a first half, a second half and not at all."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from conftest import bits
+from oracle import ops
+from test_gpu_context_attention import SPLIT_WS, _case, _check, _run
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [(1, 1), (31, 31), (32, 32), (33, 33), (2, 34), (64, 64), (65, 65), (1, 96), (30, 97), (64, 128), (5, 129)]
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("hq,hk", [(8, 2), (24, 2), (3, 1)])      # four and eight wavefronts, heads left over
+@pytest.mark.parametrize("page_size", [4, 8, 16, 32, 64])
+def test_half_step_edges(mas, dev, dim, hq, hk, page_size):
+    q_lens, kv_lens = [n for n, _ in LENGTHS], [n for _, n in LENGTHS]
+    q, kc, vc, tables, seq, cu = _case(dim + hq + page_size, q_lens, kv_lens, hq, hk, dim, page_size)
+    # Row r's keys grow (r % 3 == 1: 24-fold from position 32 on; 2: sixfold from 64 on): the reference
+    # moves in a second half, or in a later tile's first half.
+    for r, n in enumerate(kv_lens):
+        for p in range(n):
+            factor = 24.0 if r % 3 == 1 and p >= 32 else (6.0 if r % 3 == 2 and p >= 64 else 1.0)
+            kc[int(tables[r, p // page_size]), p % page_size] *= factor
+    want = ops.paged_context_attention(bits(q), bits(kc), bits(vc), tables.numpy(), seq.numpy(), cu.numpy(), 0.1)
+    for ws_bytes in (16, SPLIT_WS):
+        got = _run(mas, dev, q, kc, vc, tables, seq, cu, 0.1, ws_bytes=ws_bytes, max_kv=max(kv_lens))
+        _check(bits(got), want, min_exact=0.5)
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("hq,hk", [(8, 2), (24, 2)])
+def test_output_rows_of_ragged_tiles(mas, dev, dim, hq, hk):
+    """The last tile's tokens end inside a 32-token block: only a row's own tokens are written, in bf16
+    and fp8, into a strided view."""
+    q_lens, kv_lens = [37, 1, 70], [37, 80, 200]
+    q, kc, vc, tables, seq, cu = _case(7, q_lens, kv_lens, hq, hk, dim, 16)
+    want = ops.paged_context_attention(bits(q), bits(kc), bits(vc), tables.numpy(), seq.numpy(), cu.numpy(), 0.1)
+    tokens = sum(q_lens)
+    base = torch.full((tokens + 3, hq + 1, dim), 5.0, dtype=torch.bfloat16, device=dev)
+    _run(mas, dev, q, kc, vc, tables, seq, cu, 0.1, out=base[:tokens, 1:])
+    _check(bits(base[:tokens, 1:].contiguous()), want)
+    assert torch.all(base[tokens:] == 5.0) and torch.all(base[:, 0] == 5.0)
+    codes = torch.full((tokens + 3, hq + 1, dim), 1.0, device=dev).to(torch.float8_e4m3fn)
+    _run(mas, dev, q, kc, vc, tables, seq, cu, 0.1, out=codes[:tokens, 1:], quant=0.05)
+    y = base[:tokens, 1:].float() / 0.05
+    assert torch.equal(codes[:tokens, 1:].float(), y.clamp(-448, 448).to(torch.float8_e4m3fn).float())
+    assert torch.all(codes[tokens:].float() == 1.0) and torch.all(codes[:, 0].float() == 1.0)
