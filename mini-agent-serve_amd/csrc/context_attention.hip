@@ -33,7 +33,7 @@
 // wavefronts), and the latency of the tiles' loads. Before the halves, the unpadded LDS rows (32 DMA
 // instructions per tile for 35 or 40, no bank conflicts) and the DMA among the MFMAs, a tile's scores
 // ran beside the whole previous tile's softmax, which waited for its maximum: 4 x 4096 tokens of 96 heads
-// over 8 took 1656 us, now 1571 (1050 TFLOP/s; a large bf16 matrix product reaches 1537 on this card);
+// over 8 took 1656 us, then 1571 (1050 TFLOP/s; a large bf16 matrix product reaches 1537 on this card);
 // 4 x 2048 of 32 heads 158 -> 150 us, 6 ragged prompts after cached ones 206 -> 191 us.
 #include <algorithm>
 
@@ -950,7 +950,13 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
         s_odd = mfma32(key_op(0, 1, ks), qb[ks], s_odd);
       }
       mask(s_even, it_begin * kTileP);
-      l_run = move_reference(s_even, pb_even);
+      mask(s_odd, it_begin * kTileP + 32);
+      // The rows' first reference: the maximum over the whole tile (over its first half alone, fewer rows
+      // keep their largest p at an exact 1 and the outputs' error is 1% larger).
+#pragma unroll
+      for (int j = 0; j < 16; ++j) m_run = fmaxf(m_run, fmaxf(s_even[j], s_odd[j]));
+      m_run = fmaxf(m_run, __shfl_xor(m_run, 32));
+      l_run = weigh(s_even, (m_run == kNegInf ? 0.f : m_run) * c, pb_even);
     }
   }
   // One tile in value buffer `buf`: its second half's weights and both halves' P.V, and the next tile's
@@ -1022,48 +1028,81 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
 
   if (!wave_live) return;
   l_run += __shfl_xor(l_run, 32);  // the row's sum: both halves' shares
-  const int t = tok + n;
-  if (t >= q_len) return;
+  // ---- Output. A lane holds 4-column pieces of its token's row, so stores straight from the registers
+  // would touch 32 rows per instruction: they took 2.3 us of a workgroup's 36 at 4 x 2048 tokens of 32
+  // heads. The rows go through LDS instead, OC 16-byte chunks of each at a time (chunk c in slot c ^ a
+  // function of the row, for the banks), and leave as whole rows or halves of them, 16 bytes a lane: 150
+  // -> 143 us there, 32 x 512 tokens 130 -> 123 us, 128 tokens after 4096, whose partials go this way
+  // too, 26.9 -> 25.4 us. The key buffers hold nothing since the last tile's scores: each wavefront
+  // takes its share of them, so no barrier is needed.
+  constexpr int OC = 4 * CPR / kCtxWaves;
+  uint16_t* o_lds = (wave < kCtxWaves / 2 ? k_lds0 : k_lds1) + (wave % (kCtxWaves / 2)) * (32 * OC * 8);
+  const auto o_slot = [](int r, int ch) { return (r * OC + (ch ^ ((r / (16 / OC)) & (OC - 1)))) * 8; };
+  auto put_rows = [&](auto&& chunk_store) {  // chunk_store(token, chunk of the pass, its 16 bytes)
+    wave_lds_sync();
+#pragma unroll
+    for (int u = 0; u < OC / 2; ++u) {
+      const int r = (64 * u + lane) / OC, ch = lane % OC;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(o_lds + o_slot(r, ch));
+      if (tok + r < q_len) chunk_store(tok + r, ch, v);
+    }
+    wave_lds_sync();
+  };
   if (split_tile) {
-    // ---- this split's partial: O row (lane half hf holds columns 32 db + 8 q + 4 hf .. + 3) and
-    // (max, sum), both halves holding the same (max, sum)
-    const int64_t pi =
-        kPlan ? ((static_cast<int64_t>(d1[3]) * tokens_per_wg + (t - tile_tok)) * a.heads_per_wg + hsub) *
-                        ((d0[3] >> 24) & 0xff) + split
-              : ((static_cast<int64_t>(row) * a.row_tokens + t) * a.hq + h) * a.kv_splits + split;
-    float* po = a.part_o + pi * D + 4 * hf;
+    // ---- this split's partial: the O row and (max, sum), both lane halves holding the same (max, sum)
+    auto partial = [&](int t) {
+      return kPlan ? ((static_cast<int64_t>(d1[3]) * tokens_per_wg + (t - tile_tok)) * a.heads_per_wg + hsub) *
+                             ((d0[3] >> 24) & 0xff) + split
+                   : ((static_cast<int64_t>(row) * a.row_tokens + t) * a.hq + h) * a.kv_splits + split;
+    };
+    constexpr int PB = OC >= 8 ? OC / 8 : 1;  // 32-column blocks per pass (OC 4: half a block)
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
+    for (int pass = 0; pass < 2 * CPR / OC; ++pass) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const f32x16& o = acc[db];
-        *reinterpret_cast<f32x4*>(po + 32 * db + 8 * q) = f32x4{o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]};
-      }
-    if (hf == 0) *reinterpret_cast<f32x2*>(a.part_ml + pi * 2) = f32x2{m_run, l_run};
+      for (int b = 0; b < PB; ++b)
+#pragma unroll
+        for (int q = 0; q < (OC >= 8 ? 4 : 2); ++q) {
+          const int col4 = pass * OC + 8 * b + 2 * q;  // the piece's 16-byte chunk, less hf
+          const f32x16& o = acc[col4 / 8];
+          const int e = 4 * (col4 % 8 / 2);
+          *reinterpret_cast<f32x4*>(o_lds + o_slot(n, 8 * b + 2 * q + hf)) = f32x4{o[e], o[e + 1], o[e + 2], o[e + 3]};
+        }
+      put_rows([&](int t, int ch, u32x4 v) {
+        *reinterpret_cast<u32x4*>(a.part_o + partial(t) * D + 4 * (pass * OC + ch)) = v;
+      });
+    }
+    const int t = tok + n;
+    if (hf == 0 && t < q_len) *reinterpret_cast<f32x2*>(a.part_ml + partial(t) * 2) = f32x2{m_run, l_run};
     return;
   }
-  // ---- out[token][h][32 db + 8 q + 4 hf + i] = O / l * bmm2_scale (bf16), or its fp8 quantize
+  // ---- out[token][h] = O / l * bmm2_scale (bf16), or its fp8 quantize
   const float qs = a.out_fp8 ? (a.quant_scale_dev != nullptr ? *a.quant_scale_dev : a.quant_scale_host) : 1.f;
   const float rcp = 1.0f / qs;
   const float sc = l_run > 0.f ? a.out_scale / l_run : 0.f;
-  const int64_t at = static_cast<int64_t>(q0 + t) * a.out_stride + h * a.out_head_stride + 4 * hf;
 #pragma unroll
-  for (int db = 0; db < DB; ++db) {
+  for (int pass = 0; pass < CPR / OC; ++pass) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const f32x16& o = acc[db];
-      const uint32_t y0 = pack_bf16x2(o[4 * q] * sc, o[4 * q + 1] * sc);
-      const uint32_t y1 = pack_bf16x2(o[4 * q + 2] * sc, o[4 * q + 3] * sc);
-      const int64_t e = at + 32 * db + 8 * q;
+    for (int ch = 0; ch < OC; ++ch) {
+      const int at8 = pass * OC + ch;  // chunk 4 db + q of the row: this lane's half of it
+      const f32x16& o = acc[at8 / 4];
+      const int e = 4 * (at8 % 4);
+      *reinterpret_cast<u32x2*>(o_lds + o_slot(n, ch) + 4 * hf) =
+          u32x2{pack_bf16x2(o[e] * sc, o[e + 1] * sc), pack_bf16x2(o[e + 2] * sc, o[e + 3] * sc)};
+    }
+    put_rows([&](int t, int ch, u32x4 y) {
+      const int64_t at = static_cast<int64_t>(q0 + t) * a.out_stride + h * a.out_head_stride + 8 * (pass * OC + ch);
       if (a.out_fp8) {
         // the quantize the reference applies to the bf16 attention output (devstral2.py:93-95,110-111)
-        *reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(a.out) + e) =
-            fp8x4_saturate_encode(div_by_scale(bf16_lo(y0), qs, rcp), div_by_scale(bf16_hi(y0), qs, rcp),
-                                  div_by_scale(bf16_lo(y1), qs, rcp), div_by_scale(bf16_hi(y1), qs, rcp));
+        float v[8];
+        unpack8(y, v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = div_by_scale(v[e], qs, rcp);
+        *reinterpret_cast<u32x2*>(static_cast<uint8_t*>(a.out) + at) =
+            u32x2{fp8x4_saturate_encode(v[0], v[1], v[2], v[3]), fp8x4_saturate_encode(v[4], v[5], v[6], v[7])};
       } else {
-        *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.out) + e) = u32x2{y0, y1};
+        *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(a.out) + at) = y;
       }
-    }
+    });
   }
 }
 
