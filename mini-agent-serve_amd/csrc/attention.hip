@@ -8,7 +8,8 @@
 // in fp32 from the bf16 inputs, rounded once to bf16.
 //
 // Split-KV in two kernels:
-//  1. decode_attn_split - one wavefront per (kv head, split of split_len positions, row), kv heads
+//  1. decode_attn_split - one wavefront per (kv head, split of split_len positions, row), one or two
+//     per workgroup, kv heads
 //     adjacent in the grid so that the 256-byte slices of each 2 KB position block are read close
 //     together. The split is walked in steps of 32 positions with the next step's
 //     key and value loads in flight: Q.K^T on MFMA (v_mfma_f32_16x16x32_bf16; the kv head's G
@@ -130,9 +131,14 @@ __device__ __forceinline__ void store_output(const DecodeArgs& a, int b, int h, 
 __device__ __forceinline__ u32x4 attn_load_k(const uint16_t* p) { return load_cached(p); }
 __device__ __forceinline__ u32x4 attn_load_v(const uint16_t* p) { return load_stream(p); }
 
-// One wavefront per workgroup of the split kernel (kv heads of one position block in consecutive
-// workgroups); LDS traffic is ordered within the wavefront only.
-constexpr int kAttnWaves = 1;
+// Wavefronts per workgroup of the split kernel: two in large grids with an even kv head count, the
+// neighbouring kv heads of one split, else one (head_dim 256: one, for LDS). A pair reads 512 adjacent bytes of each
+// position from one CU: 64 rows of up to 8192 positions, 24B heads, 212 -> 201 us, 123B heads 226 -> 214
+// us, 28 rows 109 -> 106 us, 24 rows of up to 3000 (123B) 41.8 -> 39.7 us. A pair also holds its slots until
+// both end: with fewer than kPairItems (row, kv head, split) work items, one or two rounds of the GPU's wavefront
+// slots, that costs more (4 rows of up to 20000, 2528 items: 38.8 -> 40.0 us; four heads per workgroup:
+// 203 us, 216 us, 107 us). LDS traffic is ordered within the wavefront only.
+constexpr int64_t kPairItems = 4096;
 // Wavefronts per SIMD the split kernel's registers are capped for (two load buffers of a step each).
 constexpr int kAttnMinWaves = 2;
 
@@ -203,7 +209,7 @@ __device__ __forceinline__ void issue_step(const DecodeArgs& a, StepLoads<D>& st
   }
 }
 
-// One wavefront per (kv head, split, row); a split is split_len positions (whole chunks of 256, or
+// A wavefront per (kv head, split, row); a split is split_len positions (whole chunks of 256, or
 // 64 / 128 for small grids),
 // walked in steps of 32 with the next step's loads in flight (head_dim <= 128). Per step:
 // Q.K^T on MFMA -> online softmax (the running max, sum and O rescale live in the MFMA result
@@ -212,7 +218,7 @@ __device__ __forceinline__ void issue_step(const DecodeArgs& a, StepLoads<D>& st
 // the reduction). P enters as two bf16 terms, hi = bf16(P) and lo = bf16(P - hi), two MFMAs per
 // tile, so it keeps ~16 significant bits (one bf16 term alone rounds it to 8). O stays in
 // 4 * D / 16 accumulator registers whatever the group size.
-template <int GP, int D, bool kBig>
+template <int GP, int D, bool kBig, int kAttnWaves>
 __global__ __launch_bounds__(64 * kAttnWaves, D <= 128 ? kAttnMinWaves : 1) void decode_attn_split(DecodeArgs a) {
   constexpr int KS = D / 32;
   constexpr int DT = D / 16;               // MFMA tiles over the head dim for P.V
@@ -232,9 +238,17 @@ __global__ __launch_bounds__(64 * kAttnWaves, D <= 128 ? kAttnMinWaves : 1) void
 
   const int lane = threadIdx.x & 63;
   const int wave = wave_id_uniform();
-  const int kvh = blockIdx.x * kAttnWaves + wave;  // kv heads adjacent: one 2 KB position block
-  const int split = blockIdx.y, b = blockIdx.z;
-  if (kvh >= a.hk) return;
+  const int kvh = blockIdx.x * kAttnWaves + wave;  // kv heads adjacent (kAttnWaves divides them): one 2 KB position block
+  // Workgroups are dealt out to the XCDs, and within one to its shader engines, round-robin by id, and a
+  // row shorter than the table has only its first splits to do: with split = blockIdx.y the same few XCDs
+  // and engines would get all the work. The splits of row b are rotated by b + b / 4 instead (an odd count
+  // of splits spreads the rows by itself; the quarter keeps a count of 2 from falling in step with the 4
+  // engines): 200 rows of up to 1000 positions under a table of 8192, 125 -> 105 us; 64 rows of up to
+  // 3000, 4 kv heads, 53 -> 45 us; 100 rows of up to 400, 4 kv heads, 46 -> 29 us; 64 rows of up to 8192
+  // 217 -> 212 us.
+  const int b = blockIdx.z;
+  const unsigned turn = gridDim.y & 1 ? 0u : blockIdx.z + (blockIdx.z >> 2);
+  const int split = static_cast<int>((blockIdx.y + turn) % gridDim.y);
   uint16_t* v_lds = v_lds_all[wave];
   uint16_t(*p_lds)[16 * PROW] = p_lds_all[wave];
   int32_t* pg_lds = pg_lds_all[wave];
@@ -556,18 +570,28 @@ __global__ __launch_bounds__(64) void decode_attn_combine(DecodeArgs a) {
   store_output<DPL>(a, b, h, DPL * lane, y);
 }
 
-template <int GP, int D>
-int launch(const DecodeArgs& a, int64_t batch, int64_t hk, hipStream_t s) {
-  const dim3 grid(static_cast<uint32_t>(cdiv(hk, kAttnWaves)), static_cast<uint32_t>(a.max_splits),
+template <int GP, int D, int kAttnWaves>
+void launch_split(const DecodeArgs& a, int64_t batch, int64_t hk, hipStream_t s) {
+  const dim3 grid(static_cast<uint32_t>(hk / kAttnWaves), static_cast<uint32_t>(a.max_splits),
                   static_cast<uint32_t>(batch));
   // Pages of at least one chunk: every 32-position step lies in one page, addressed from its base
   // with 32-bit byte offsets (the largest in-page offset is checked here).
   const int64_t page_size = int64_t{1} << a.log2_page;
   const int64_t in_page = 2 * ((page_size - 1) * a.entry_stride + D);
   if (page_size >= kChunk && in_page <= INT32_MAX)
-    hipLaunchKernelGGL((decode_attn_split<GP, D, true>), grid, dim3(64 * kAttnWaves), 0, s, a);
+    hipLaunchKernelGGL((decode_attn_split<GP, D, true, kAttnWaves>), grid, dim3(64 * kAttnWaves), 0, s, a);
   else
-    hipLaunchKernelGGL((decode_attn_split<GP, D, false>), grid, dim3(64 * kAttnWaves), 0, s, a);
+    hipLaunchKernelGGL((decode_attn_split<GP, D, false, kAttnWaves>), grid, dim3(64 * kAttnWaves), 0, s, a);
+}
+
+template <int GP, int D>
+int launch(const DecodeArgs& a, int64_t batch, int64_t hk, hipStream_t s) {
+  bool pairs = false;
+  if constexpr (D <= 128) {
+    pairs = hk % 2 == 0 && batch * hk * a.max_splits >= kPairItems;
+    if (pairs) launch_split<GP, D, 2>(a, batch, hk, s);
+  }
+  if (!pairs) launch_split<GP, D, 1>(a, batch, hk, s);
   if (const int st = launch_status(); st != MAS_OK) return st;
   hipLaunchKernelGGL((decode_attn_combine<D>), dim3(static_cast<uint32_t>(a.hq), static_cast<uint32_t>(batch)),
                      dim3(64), 0, s, a);
