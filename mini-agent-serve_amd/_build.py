@@ -1,5 +1,5 @@
-"""Build recipe for libmas_kernels.so, the C-ABI library of the gfx950 layer kernels, and for
-libmas_bench.so, the benchmark's memory skeletons.
+"""Build recipe for libmas_kernels.so, the C-ABI library of the gfx950 layer kernels, for
+direct_calls.so, the Python calls into it, and for libmas_bench.so, the benchmark's memory skeletons.
 
 Every ``csrc/*.hip`` file is compiled for gfx950 with hipcc (in parallel), then linked into one
 shared library next to this file; ``bench_csrc/*.hip`` likewise into the benchmark's library. The
@@ -11,6 +11,7 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
@@ -22,6 +23,8 @@ INCLUDE_DIR = PACKAGE_DIR.parent / "include"
 LIBRARY_NAME = "libmas_kernels.so"
 LIBRARY_PATH = PACKAGE_DIR / LIBRARY_NAME
 BENCH_LIBRARY_PATH = PACKAGE_DIR / "libmas_bench.so"
+DIRECT_CALLS_SOURCE = PACKAGE_DIR / "binding" / "direct_calls.cpp"
+DIRECT_CALLS_PATH = PACKAGE_DIR / "direct_calls.so"
 ARCH = "gfx950"
 
 # -ffp-contract=off keeps every fp32 product and sum separately rounded, so the kernels' arithmetic
@@ -85,6 +88,28 @@ def build_library(verbose: bool = False, jobs: int | None = None, directory: Pat
     return library
 
 
+def build_direct_calls(verbose: bool = False) -> Path:
+    """Compiles the Python extension that checks a layer's tensors and calls the kernel library (host
+    code only, against torch's own headers and libraries)."""
+    import torch
+
+    root = Path(torch.__path__[0])
+    hip_include = Path(hipcc()).resolve().parent.parent / "include"
+    staged = DIRECT_CALLS_PATH.parent / f".{DIRECT_CALLS_PATH.name}.tmp{os.getpid()}"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{root / 'include'}",
+           f"-I{root / 'include' / 'torch' / 'csrc' / 'api' / 'include'}", f"-I{sysconfig.get_paths()['include']}",
+           f"-isystem{hip_include}", "-isystem/opt/rocm/include", str(DIRECT_CALLS_SOURCE), "-o", str(staged),
+           f"-L{root / 'lib'}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"{DIRECT_CALLS_SOURCE.name} failed:\n{' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
+    os.replace(staged, DIRECT_CALLS_PATH)
+    if verbose:
+        print(f"built {DIRECT_CALLS_PATH}")
+    return DIRECT_CALLS_PATH
+
+
 def build_bench_library(verbose: bool = False) -> Path:
     """The benchmark's memory skeletons (not part of the kernel library)."""
     return build_library(verbose, directory=BENCH_CSRC_DIR, library=BENCH_LIBRARY_PATH)
@@ -92,4 +117,5 @@ def build_bench_library(verbose: bool = False) -> Path:
 
 if __name__ == "__main__":
     build_library(verbose=True)
+    build_direct_calls(verbose=True)
     build_bench_library(verbose=True)

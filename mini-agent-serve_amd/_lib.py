@@ -8,6 +8,7 @@ machine without the built library every op raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import threading
 
 import torch  # noqa: F401  (must precede the CDLL load, see above)
@@ -71,17 +72,37 @@ ERROR_BITS = {
     32: "placeholder -1 - r past the previous step's samples",
 }
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
+
+# The extension of binding/direct_calls.cpp, bound to the library: set by load(). Its functions return
+# the C entry point's status, or None for a form they do not take, which the wrappers then handle.
+direct = None
 
 
 class KernelError(RuntimeError):
     """A nonzero status returned by the kernel library."""
 
 
+def _load_direct(lib: ctypes.CDLL):
+    path = _build.DIRECT_CALLS_PATH
+    if not path.exists():
+        raise RuntimeError(
+            f"{path.name} is not built (expected at {path}); build it with "
+            "`python -c 'import __graft_entry__ as g; g.build()'` from the repository root")
+    spec = importlib.util.spec_from_file_location("direct_calls", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    if _raw_stream is None:
+        return None
+    module.bind(_raw_stream, {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _SIGNATURES})
+    return module
+
+
 def load() -> ctypes.CDLL:
     """Returns the loaded library, loading it on first use."""
-    global _lib
+    global _lib, direct
     if _lib is not None:
         return _lib
     with _lock:
@@ -96,6 +117,7 @@ def load() -> ctypes.CDLL:
                 fn = getattr(lib, name)
                 fn.argtypes = argtypes
                 fn.restype = _RESTYPES.get(name, ctypes.c_int)
+            direct = _load_direct(lib)
             _lib = lib
     return _lib
 
@@ -112,9 +134,6 @@ def check(status: int, what: str) -> None:
 
 def describe_error_bits(bits: int) -> str:
     return "; ".join(text for bit, text in ERROR_BITS.items() if bits & bit) or "none"
-
-
-_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def stream_handle(device: torch.device) -> int:

@@ -47,6 +47,10 @@ def silu_and_mul(input: torch.Tensor, out: torch.Tensor | None = None, enable_pd
         return out
     if out is None:
         out = torch.empty(tuple(input.shape[:-1]) + (input.shape[-1] // 2,), dtype=input.dtype, device=input.device)
+    if _lib.direct is not None and (st := _lib.direct.silu_and_mul(input, out)) is not None:
+        if st:
+            _lib.check(st, "silu_and_mul")
+        return out
     _silu_and_mul(input, out)
     return out
 
@@ -96,5 +100,9 @@ def silu_and_mul_quant(input: torch.Tensor, scale: torch.Tensor | float, out: to
         return out
     if out is None:
         out = torch.empty(tuple(input.shape[:-1]) + (input.shape[-1] // 2,), dtype=FP8, device=input.device)
+    if _lib.direct is not None and (st := _lib.direct.silu_and_mul_quant(input, out, scale)) is not None:
+        if st:
+            _lib.check(st, "silu_and_mul_quant")
+        return out
     _silu_and_mul_quant(input, out, scale)
     return out

@@ -173,6 +173,12 @@ def trtllm_batch_decode_with_kv_cache(query: torch.Tensor, kv_cache, workspace_b
                                              float(bmm1_scale), float(bmm2_scale), out, kv_layout, qs, qs_host,
                                              error_flags)
         return out
+    if _lib.direct is not None and (st := _lib.direct.decode_attention(
+            query, kv_cache, workspace_buffer, block_tables, seq_lens, bmm1_scale, bmm2_scale, out, kv_layout,
+            error_flags, out_quant_scale)) is not None:
+        if st:
+            _lib.check(st, "trtllm_batch_decode_with_kv_cache")
+        return out
     _decode(query, kv_cache, workspace_buffer, block_tables, seq_lens, bmm1_scale, bmm2_scale, out, kv_layout,
             error_flags, out_quant_scale)
     return out
@@ -269,6 +275,12 @@ def trtllm_batch_context_with_kv_cache(query: torch.Tensor, kv_cache, workspace_
         torch.ops.mas.paged_context_attention(query, k_cache, v_cache, workspace_buffer, block_tables, seq_lens,
                                               cum_seq_lens_q, int(max_q_len), int(max_kv_len), float(bmm1_scale),
                                               float(bmm2_scale), out, kv_layout, qs, qs_host, error_flags)
+        return out
+    if _lib.direct is not None and (st := _lib.direct.context_attention(
+            query, kv_cache, workspace_buffer, block_tables, seq_lens, cum_seq_lens_q, max_q_len, max_kv_len,
+            bmm1_scale, bmm2_scale, out, kv_layout, error_flags, out_quant_scale)) is not None:
+        if st:
+            _lib.check(st, "trtllm_batch_context_with_kv_cache")
         return out
     _context(query, kv_cache, block_tables, seq_lens, cum_seq_lens_q, max_q_len, bmm1_scale, bmm2_scale, out,
              kv_layout, error_flags, out_quant_scale, workspace_buffer, max_kv_len)

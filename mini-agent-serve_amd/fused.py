@@ -122,5 +122,23 @@ def apply_rope_and_append_paged_kv_cache(positions: torch.Tensor, query: torch.T
                                                            float(llama_4_scaling_beta),
                                                            int(original_max_position_embeddings), error_flags)
         return
+    if _lib.direct is not None:
+        q_scale, interval = None, 0
+        ready = True
+        if llama_4_scaling_beta:  # a table made by an earlier call, as _fused asks for it; else its way
+            ready = (isinstance(original_max_position_embeddings, int) and original_max_position_embeddings > 0
+                     and type(cos_sin_cache) is torch.Tensor and cos_sin_cache.dim() == 2
+                     and isinstance(query, torch.Tensor))
+            if ready:
+                interval = original_max_position_embeddings
+                q_scale = _Q_SCALE_TABLES.get((float(llama_4_scaling_beta), interval,
+                                               max(-(-cos_sin_cache.shape[0] // interval), 1), query.device))
+                ready = q_scale is not None
+        if ready and (st := _lib.direct.rope_append(
+                positions, query, key, value, head_size, cos_sin_cache, is_neox, batch_indices, paged_kv_cache,
+                kv_indices, kv_indptr, kv_layout, error_flags, q_scale, interval)) is not None:
+            if st:
+                _lib.check(st, "apply_rope_and_append_paged_kv_cache")
+            return
     _fused(positions, query, key, value, head_size, cos_sin_cache, is_neox, batch_indices, paged_kv_cache,
            kv_indices, kv_indptr, kv_layout, error_flags, llama_4_scaling_beta, original_max_position_embeddings)

@@ -81,6 +81,10 @@ def fused_add_rmsnorm(input: torch.Tensor, residual: torch.Tensor, weight: torch
     if torch.compiler.is_compiling():
         torch.ops.mas.fused_add_rmsnorm(input, residual, weight, float(eps))
         return
+    if _lib.direct is not None and (st := _lib.direct.fused_add_rmsnorm(input, residual, weight, eps)) is not None:
+        if st:
+            _lib.check(st, "fused_add_rmsnorm")
+        return
     _fused_add_rmsnorm(input, residual, weight, eps)
 
 
@@ -96,5 +100,9 @@ def fused_add_rmsnorm_quant(out: torch.Tensor, input: torch.Tensor, residual: to
             torch.ops.mas.fused_add_rmsnorm_quant(out, input, residual, weight, scale, float(eps))
         else:
             torch.ops.mas.fused_add_rmsnorm_quant_hs(out, input, residual, weight, float(scale), float(eps))
+        return
+    if _lib.direct is not None and (st := _lib.direct.fused_add_rmsnorm_quant(out, input, residual, weight, scale, eps)) is not None:
+        if st:
+            _lib.check(st, "fused_add_rmsnorm_quant")
         return
     _fused_add_rmsnorm_quant(out, input, residual, weight, scale, eps)
