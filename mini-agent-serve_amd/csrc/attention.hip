@@ -494,21 +494,28 @@ __global__ __launch_bounds__(64) void decode_attn_combine(DecodeArgs a) {
 #pragma unroll
   for (int e = 0; e < DPL; ++e) acc[e] = 0.f;
   float lsum = 0.f;
-  constexpr int kOneRound = 32;
+  constexpr int kOneRound = 32, kGroup = 8;
   if (nsplit <= kOneRound) {
     // Every load in one round trip: lane s reads split s's (max, sum), and all splits' partial O
-    // rows are loaded (indices past the last split clamped to it, weighted 0) before the max is
-    // known. Same weights and summation order as the general path below.
-    const int sl = lane < nsplit ? lane : (nsplit > 0 ? nsplit - 1 : 0);
+    // rows are loaded, in groups of 8 as far as the row's splits go (indices past the last split
+    // clamped to it, weighted 0), before the max is known. Same weights and summation order as the general path below.
+    const int last = nsplit > 0 ? nsplit - 1 : 0;
+    const int sl = lane < nsplit ? lane : last;
     const f32x2 ml = *reinterpret_cast<const f32x2*>(a.part_ml + (base + sl) * 2);
     const float* po = a.part_o + base * D + DPL * lane;
     float v[kOneRound][DPL];
+    auto load_group = [&](int u0) {
 #pragma unroll
-    for (int u = 0; u < kOneRound; ++u) {
-      const int su = u < nsplit ? u : sl;
+      for (int u = u0; u < u0 + kGroup; ++u) {
+        const int su = u < nsplit ? u : last;
 #pragma unroll
-      for (int e = 0; e < DPL; ++e) v[u][e] = po[su * D + e];
-    }
+        for (int e = 0; e < DPL; ++e) v[u][e] = po[su * D + e];
+      }
+    };
+    load_group(0);
+#pragma unroll
+    for (int u0 = kGroup; u0 < kOneRound; u0 += kGroup)
+      if (nsplit > u0) load_group(u0);  // uniform
     const float m_lane = lane < nsplit ? ml[0] : kNegInf;
     const float mx = wave_max(m_lane);
     if (mx != kNegInf) {
