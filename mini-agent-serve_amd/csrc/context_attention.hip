@@ -46,7 +46,7 @@ constexpr int kTileP = 64;        // key positions per tile
 constexpr int kRowsPerWave = 32;  // query rows (tokens of one head) per wavefront
 constexpr int kMaxCtxSplits = 32;  // split-KV: key-range splits per token tile, at most
 constexpr float kNegInf = -__builtin_huge_valf();
-// The online softmax's lazy reference point: a half tile's p = 2^(s c - m c) sum to at most this per lane.
+// The online softmax's lazy reference point: a tile's p = 2^(s c - m c) sum to at most this per lane.
 constexpr float kSumMost = 256.f;
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -667,7 +667,8 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
     return;
   }
 
-  float m_run = kNegInf, l_run = 0.f;  // token n's running max (raw score units) and this half's sum
+  // token n's softmax reference (raw score units), and this lane's sums: the tiles so far, this tile so far
+  float m_run = kNegInf, l_run = 0.f, t_run = 0.f;
   f32x16 acc[DB];                      // O^T: element j of block db holds O[token n][32 db + 8 (j/4) + 4 hf + j%4]
 #pragma unroll
   for (int db = 0; db < DB; ++db) acc[db] = f32x16{};
@@ -827,16 +828,15 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   //            16 kk + 8 + 4 hf + e - 4 (e >= 4), i.e. elements 8 kk .. + 7 of s;
   //   pv     - O^T += V^T P^T: A = V^T[32 dims][16 positions], read transposed from the row-major
   //            value tile in that position order.
-  auto key_op = [&](int buf, int half, int ks) {
-    return *reinterpret_cast<const bf16x8*>(klds(buf) + 32 * half * D + (key_at0 ^ 16 * ks));
+  auto key_op = [&](int buf, int half, int ks, int at0) {
+    return *reinterpret_cast<const bf16x8*>(klds(buf) + 32 * half * D + (at0 ^ 16 * ks));
   };
-  auto value_op = [&](int buf, int kk, int db) {
-    const uint16_t* p = vlds(buf) + 16 * kk * D + (value_at0 ^ 32 * db);
+  auto value_op = [&](int buf, int kk, int db, int at0) {
+    const uint16_t* p = vlds(buf) + 16 * kk * D + (at0 ^ 32 * db);
     const i16x4 lo = read_transposed4(p), hi = read_transposed4(p + 8 * D);
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  auto weigh = [&](const f32x16& s, float mc, bf16x8 (&pbo)[2]) {
-    float sum = 0.f;
+  auto weigh = [&](const f32x16& s, float mc, float sum, bf16x8 (&pbo)[2]) {
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
       float p[8];
@@ -849,7 +849,7 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
                             pack_bf16x2(p[6], p[7])};
       pbo[kk] = __builtin_bit_cast(bf16x8, packed);
     }
-    return sum;  // this lane's share: half of the row's 32
+    return sum;  // the sum it was given, and this lane's share of the half: 16 of the row's 32
   };
   // ---- causal mask, only on halves that cross the diagonal of the wavefront's first row or the end
   // of the sequence (a wavefront-uniform branch)
@@ -865,13 +865,14 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   };
   // ---- online softmax per query row; scores stay in raw units, the scale enters the exponent
   // through one fma. The reference point m is lazy: a half's p are taken against the m its row has,
-  // and only where a lane's 16 p sum to more than kSumMost does the wavefront move its rows' m to the
-  // maximum of their scores, rescale O and l, and take the half's p again. p stays below kSumMost, and
-  // bf16 P and the fp32 sums carry the same relative precision at any such magnitude; O / l does not
-  // depend on m. A row's first scores find m = -inf: their p are +inf (NaN for a masked score), which
-  // the test catches as well. The split partials carry this m with their sums. Each lane keeps its
-  // share of the sum in l_run; the two lanes of a row add theirs after the last tile.
-  auto move_reference = [&](const f32x16& s, bf16x8 (&pbo)[2]) {
+  // and only where a lane's p of the tile so far sum to more than kSumMost does the wavefront move its
+  // rows' m to the maximum of their scores, rescale O and the sums, and take the half's p again. p stays
+  // below kSumMost, and bf16 P and the fp32 sums carry the same relative precision at any such magnitude;
+  // O / l does not depend on m. A row's first scores find m = -inf: their p are +inf (NaN for a masked
+  // score), which the test catches as well. The split partials carry this m with their sums. A lane adds
+  // its 32 p of a tile in one chain, t_run over its first half, and each tile's sum to l_run; the two
+  // lanes of a row add theirs after the last tile.
+  auto move_reference = [&](const f32x16& s, bool second, bf16x8 (&pbo)[2]) {
     float mh = kNegInf;
 #pragma unroll
     for (int j = 0; j < 16; ++j) mh = fmaxf(mh, s[j]);
@@ -881,14 +882,18 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
     m_run = m_new;
     if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
       l_run *= alpha;
+      t_run *= alpha;
 #pragma unroll
       for (int db = 0; db < DB; ++db) acc[db] *= alpha;
     }
-    return weigh(s, (m_run == kNegInf ? 0.f : m_run) * c, pbo);
+    return weigh(s, (m_run == kNegInf ? 0.f : m_run) * c, second ? t_run : 0.f, pbo);
   };
-  auto settle = [&](float sum, const f32x16& s, bf16x8 (&pbo)[2]) {
-    if (__builtin_amdgcn_ballot_w64(!(sum <= kSumMost)) != 0) sum = move_reference(s, pbo);  // wavefront-uniform
-    l_run += sum;
+  // The weights of a tile's first or second half against the row's m, which moves where it must.
+  auto weigh_half = [&](const f32x16& s, bool second, bf16x8 (&pbo)[2]) {
+    float sum = weigh(s, m_run * c, second ? t_run : 0.f, pbo);
+    if (__builtin_amdgcn_ballot_w64(!(sum <= kSumMost)) != 0) sum = move_reference(s, second, pbo);  // wavefront-uniform
+    if (second) l_run += sum;
+    else t_run = sum;
   };
   // One half's work, the three parts of three different halves, so that none waits for another: the
   // scores of half h + 1 (key half `khalf` of buffer kbuf) into `nxt`, the weights of half h (`cur`,
@@ -896,17 +901,21 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   // MFMAs alternate (a half's scores are one chain over the head dim), with the reads of the operands
   // ahead of them and the weights' instructions between them.
   auto half_step = [&](int kbuf, int khalf, f32x16& nxt, int vbuf, int vhalf, const bf16x8 (&pb_prev)[2],
-                       const f32x16& cur, bf16x8 (&pb_cur)[2], auto&& load) {
+                       const f32x16& cur, bool second, bf16x8 (&pb_cur)[2], auto&& load) {
     f32x16 sn{};
+    int key_at = key_at0, value_at = value_at0;
+    // kPagesLane with four wavefronts, a tile in registers besides: the copies keep the compiler from holding
+    // all 12 read addresses over the loop (2 x 64 tokens after 3000, 4-slot pages, 28.5 -> 26.8 us; 500 after
+    // 500 32.9 -> 30.3 us).
+    if constexpr (!kDirect && kWaves == 4) asm volatile("" : "+v"(key_at), "+v"(value_at));
 #pragma unroll
     for (int i = 0; i < KS; ++i) {
-      sn = mfma32(key_op(kbuf, khalf, i), qb[i], sn);
-      acc[i % DB] = mfma32(value_op(vbuf, 2 * vhalf + i / DB, i % DB), pb_prev[i / DB], acc[i % DB]);
+      sn = mfma32(key_op(kbuf, khalf, i, key_at), qb[i], sn);
+      acc[i % DB] = mfma32(value_op(vbuf, 2 * vhalf + i / DB, i % DB, value_at), pb_prev[i / DB], acc[i % DB]);
       load(i);
     }
-    const float sum = weigh(cur, m_run * c, pb_cur);
+    weigh_half(cur, second, pb_cur);
     nxt = sn;
-    settle(sum, cur, pb_cur);
   };
 
   TileRegs tr;
@@ -946,8 +955,8 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
     if (wave_live) {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        s_even = mfma32(key_op(0, 0, ks), qb[ks], s_even);
-        s_odd = mfma32(key_op(0, 1, ks), qb[ks], s_odd);
+        s_even = mfma32(key_op(0, 0, ks, key_at0), qb[ks], s_even);
+        s_odd = mfma32(key_op(0, 1, ks, key_at0), qb[ks], s_odd);
       }
       mask(s_even, it_begin * kTileP);
       mask(s_odd, it_begin * kTileP + 32);
@@ -956,7 +965,7 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
 #pragma unroll
       for (int j = 0; j < 16; ++j) m_run = fmaxf(m_run, fmaxf(s_even[j], s_odd[j]));
       m_run = fmaxf(m_run, __shfl_xor(m_run, 32));
-      l_run = weigh(s_even, (m_run == kNegInf ? 0.f : m_run) * c, pb_even);
+      t_run = weigh(s_even, (m_run == kNegInf ? 0.f : m_run) * c, 0.f, pb_even);
     }
   }
   // One tile in value buffer `buf`: its second half's weights and both halves' P.V, and the next tile's
@@ -986,9 +995,9 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
     };
     if (wave_live) {
       mask(s_odd, it * kTileP + 32);
-      half_step(buf ^ 1, 0, s_even, buf, 0, pb_even, s_odd, pb_odd, load_value);
+      half_step(buf ^ 1, 0, s_even, buf, 0, pb_even, s_odd, true, pb_odd, load_value);
       mask(s_even, (it + 1) * kTileP);
-      half_step(buf ^ 1, 1, s_odd, buf, 1, pb_odd, s_even, pb_even, load_key);
+      half_step(buf ^ 1, 1, s_odd, buf, 1, pb_odd, s_even, false, pb_even, load_key);
     } else if constexpr (kDirect) {
       dma_values(value_pages, vlds(buf ^ 1));
       dma_keys(ahead, klds(buf));
@@ -1000,14 +1009,16 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
     if (wave_live) {
       auto pv = [&](int half, const bf16x8 (&pb)[2]) {
 #pragma unroll
-        for (int i = 0; i < KS; ++i) acc[i % DB] = mfma32(value_op(buf, 2 * half + i / DB, i % DB), pb[i / DB], acc[i % DB]);
+        for (int i = 0; i < KS; ++i)
+          acc[i % DB] = mfma32(value_op(buf, 2 * half + i / DB, i % DB, value_at0), pb[i / DB], acc[i % DB]);
       };
       mask(s_odd, it * kTileP + 32);
       pv(0, pb_even);
-      if (it * kTileP + 32 <= shift + tok + kRowsPerWave - 1) {  // else no row sees the second half
-        const float sum = weigh(s_odd, m_run * c, pb_odd);
-        settle(sum, s_odd, pb_odd);
+      if (it * kTileP + 32 <= shift + tok + kRowsPerWave - 1) {
+        weigh_half(s_odd, true, pb_odd);
         pv(1, pb_odd);
+      } else {  // no row sees the second half
+        l_run += t_run;
       }
     }
   };

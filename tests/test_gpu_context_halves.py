@@ -51,3 +51,27 @@ def test_output_rows_of_ragged_tiles(mas, dev, dim, hq, hk):
     y = base[:tokens, 1:].float() / 0.05
     assert torch.equal(codes[:tokens, 1:].float(), y.clamp(-448, 448).to(torch.float8_e4m3fn).float())
     assert torch.all(codes[tokens:].float() == 1.0) and torch.all(codes[:, 0].float() == 1.0)
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("tiles", [1, 2, 3, 4])
+@pytest.mark.parametrize("page_size", [4, 16, 64])
+def test_a_tiles_weights_add_in_one_chain(mas, dev, dim, tiles, page_size):
+    """A lane adds its 32 weights of a 64-position tile one after the other, over both halves. Every tile has
+    one weight of 1 (value 1) in a lane's first half and 16 of 2^-25 (value 0) in its second: each vanishes
+    beside the 1, so the row's sum is the number of tiles, and an output scaled to 2^-22 above the middle of
+    two bf16 values rounds up. The 16 added by themselves would make 2^-21 of each tile, and it would round
+    down (the key's bf16 rounding moves 2^-25 by at most 2^0.15)."""
+    scale, n = 0.1, 64 * tiles
+    small = -25 / (scale * 1.4426950408889634)
+    q, kc, vc, tables, seq, cu = _case(1, [1], [n], 4, 1, dim, page_size)
+    q.zero_()
+    q[..., 0] = 1
+    kc.zero_()
+    vc.zero_()
+    for p in range(n):
+        at = int(tables[0, p // page_size]), p % page_size, 0
+        kc[at][0] = 0.0 if p % 64 == 0 else (small if p % 64 >= 32 and p % 8 < 4 else -20000.0)
+        vc[at] = 1.0 if p % 64 == 0 else 0.0
+    got = _run(mas, dev, q, kc, vc, tables, seq, cu, scale, scale2=1 + 2 ** -8 + 2 ** -22)
+    assert torch.all(got == 1 + 2 ** -7), got.unique()
