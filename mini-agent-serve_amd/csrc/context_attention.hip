@@ -865,20 +865,24 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   };
   // ---- online softmax per query row; scores stay in raw units, the scale enters the exponent
   // through one fma. The reference point m is lazy: a half's p are taken against the m its row has,
-  // and only where a lane's p of the tile so far sum to more than kSumMost does the wavefront move its
-  // rows' m to the maximum of their scores, rescale O and the sums, and take the half's p again. p stays
-  // below kSumMost, and bf16 P and the fp32 sums carry the same relative precision at any such magnitude;
-  // O / l does not depend on m. A row's first scores find m = -inf: their p are +inf (NaN for a masked
-  // score), which the test catches as well. The split partials carry this m with their sums. A lane adds
+  // and only a row where a lane's p of the tile so far sum to more than kSumMost moves its m to the
+  // maximum of its scores; the wavefront then rescales O and the sums and takes the half's p again (the
+  // other rows' by 1 and to the same bits: a token's output does not depend on its tile's other tokens). p
+  // stays below kSumMost, and bf16 P and the fp32 sums carry the same relative precision at any such
+  // magnitude; O / l does not depend on m. A row's first scores find m = -inf: their p are +inf (NaN for a
+  // masked score), which the test catches as well. The split partials carry this m with their sums. A lane adds
   // its 32 p of a tile in one chain, t_run over its first half, and each tile's sum to l_run; the two
   // lanes of a row add theirs after the last tile.
-  auto move_reference = [&](const f32x16& s, bool second, bf16x8 (&pbo)[2]) {
+  auto move_reference = [&](const f32x16& s, bool second, bool over, bf16x8 (&pbo)[2]) {
     float mh = kNegInf;
 #pragma unroll
     for (int j = 0; j < 16; ++j) mh = fmaxf(mh, s[j]);
-    const float m_new = fmaxf(m_run, fmaxf(mh, __shfl_xor(mh, 32)));  // the same in both lanes
-    // rows that had no finite score have O = 0 and l = 0: their factor is 1
-    const float alpha = m_run != kNegInf ? __builtin_amdgcn_exp2f(__builtin_fmaf(m_run, c, -(m_new * c))) : 1.f;
+    const float mx = fmaxf(mh, __shfl_xor(mh, 32));  // the same in both lanes of a row, either of which moves it
+    const bool moves = (__shfl_xor(over ? 1 : 0, 32) | (over ? 1 : 0)) != 0;
+    const float m_new = moves ? fmaxf(m_run, mx) : m_run;
+    // rows that had no finite score have O = 0 and l = 0: their factor is 1, as that of a row that stays is
+    // (m c - m c rounded is not 0)
+    const float alpha = moves && m_run != kNegInf ? __builtin_amdgcn_exp2f(__builtin_fmaf(m_run, c, -(m_new * c))) : 1.f;
     m_run = m_new;
     if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
       l_run *= alpha;
@@ -891,7 +895,8 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   // The weights of a tile's first or second half against the row's m, which moves where it must.
   auto weigh_half = [&](const f32x16& s, bool second, bf16x8 (&pbo)[2]) {
     float sum = weigh(s, m_run * c, second ? t_run : 0.f, pbo);
-    if (__builtin_amdgcn_ballot_w64(!(sum <= kSumMost)) != 0) sum = move_reference(s, second, pbo);  // wavefront-uniform
+    const bool over = !(sum <= kSumMost);
+    if (__builtin_amdgcn_ballot_w64(over) != 0) sum = move_reference(s, second, over, pbo);  // wavefront-uniform
     if (second) l_run += sum;
     else t_run = sum;
   };

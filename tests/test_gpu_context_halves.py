@@ -75,3 +75,22 @@ def test_a_tiles_weights_add_in_one_chain(mas, dev, dim, tiles, page_size):
         vc[at] = 1.0 if p % 64 == 0 else 0.0
     got = _run(mas, dev, q, kc, vc, tables, seq, cu, scale, scale2=1 + 2 ** -8 + 2 ** -22)
     assert torch.all(got == 1 + 2 ** -7), got.unique()
+
+
+@pytest.mark.parametrize("page_size,kv_len,ws_bytes", [(4, 320, 16), (16, 320, 16), (64, 320, 16), (16, 1600, SPLIT_WS)])
+@pytest.mark.parametrize("dim,hq,hk", [(64, 8, 2), (128, 8, 2), (128, 24, 2)])
+def test_outputs_do_not_depend_on_the_tiles_other_tokens(mas, dev, dim, hq, hk, page_size, kv_len, ws_bytes):
+    """Odd tokens' scores grow so that their softmax reference moves in every tile, or are nearly flat so that
+    it never does: the even tokens between them, whose own scores rise a little, get the same bits."""
+    q_len = 60
+    q, kc, vc, tables, seq, cu = _case(dim + hq + kv_len, [q_len], [kv_len], hq, hk, dim, page_size)
+    for p in range(64, kv_len):
+        kc[int(tables[0, p // page_size]), p % page_size] *= 1 + p / kv_len
+    got = []
+    for factor in (30.0, 0.01):
+        mixed = q.clone()
+        mixed[1::2] *= factor
+        got.append(_run(mas, dev, mixed, kc, vc, tables, seq, cu, 0.1, ws_bytes=ws_bytes, max_kv=kv_len))
+    assert torch.equal(got[0][0::2], got[1][0::2])
+    want = ops.paged_context_attention(bits(mixed), bits(kc), bits(vc), tables.numpy(), seq.numpy(), cu.numpy(), 0.1)
+    _check(bits(got[1]), want, min_exact=0.5)
