@@ -94,3 +94,21 @@ def test_outputs_do_not_depend_on_the_tiles_other_tokens(mas, dev, dim, hq, hk, 
     assert torch.equal(got[0][0::2], got[1][0::2])
     want = ops.paged_context_attention(bits(mixed), bits(kc), bits(vc), tables.numpy(), seq.numpy(), cu.numpy(), 0.1)
     _check(bits(got[1]), want, min_exact=0.5)
+
+
+@pytest.mark.parametrize("dim,hq,hk", [(64, 4, 1), (128, 4, 1), (128, 5, 1), (128, 12, 1)])  # four, then eight wavefronts
+@pytest.mark.parametrize("page_size", [4, 8, 16, 32, 64, 256])
+def test_split_ranges_end_at_every_half(mas, dev, dim, hq, hk, page_size):
+    """Rows of 17 and 18 key tiles under a table of 64, which gives ranges of 4: the last range is one or two
+    tiles long and ends at, before and after a tile's middle. The workspace tells that the launch was split."""
+    q_lens = [1, 31, 32, 33, 2, 30, 32, 5]
+    kv_lens = [1024 + n for n in (1, 31, 32, 33, 64, 65, 96, 97)]
+    q, kc, vc, tables, seq, cu = _case(hq + dim + page_size, q_lens, kv_lens, hq, hk, dim, page_size)
+    tables = torch.nn.functional.pad(tables, (0, 4096 // page_size - tables.shape[1]))
+    ws = torch.full((SPLIT_WS,), 255, dtype=torch.uint8, device=dev)
+    got = mas.attention.trtllm_batch_context_with_kv_cache(
+        q.to(dev), (kc.to(dev), vc.to(dev)), ws, tables.to(dev), seq.to(dev), 33, 4096, dim ** -0.5, 1.0, len(q_lens),
+        cu.to(dev))
+    assert not torch.all(ws == 255)
+    want = ops.paged_context_attention(bits(q), bits(kc), bits(vc), tables.numpy(), seq.numpy(), cu.numpy(), dim ** -0.5)
+    _check(bits(got), want, min_exact=0.5)
