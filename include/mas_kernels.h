@@ -56,7 +56,9 @@ extern "C" {
 #define MAS_ERRBIT_SLOT 16u     /* kv slot form: slot >= num_pages * page_size            */
 #define MAS_ERRBIT_PLACEHOLDER 32u /* embedding: placeholder -1 - r with r >= num_last     */
 
-/* Library version, (major << 16) | (minor << 8) | patch. */
+/* Library version, (major << 16) | (minor << 8) | patch: of this header, and of the library loaded. A
+   change to a function's signature or to a constant's meaning changes it. */
+#define MAS_VERSION ((0 << 16) | (1 << 8) | 0)
 int mas_version(void);
 
 /* Human-readable text for a return code of this library. */

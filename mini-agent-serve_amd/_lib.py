@@ -9,7 +9,9 @@ from __future__ import annotations
 
 import ctypes
 import importlib.util
+import sys
 import threading
+import warnings
 
 import torch  # noqa: F401  (must precede the CDLL load, see above)
 
@@ -76,8 +78,9 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
 
-# The extension of binding/direct_calls.cpp, bound to the library: set by load(). Its functions return
-# the C entry point's status, or None for a form they do not take, which the wrappers then handle.
+# The extension of binding/direct_calls.cpp, bound to the library: set by load(), None where it is not there
+# or not built for this torch, Python and library (the wrappers then take every call). Its functions
+# return the C entry point's status, or None for a form they do not take, which the wrappers then handle.
 direct = None
 
 
@@ -86,17 +89,22 @@ class KernelError(RuntimeError):
 
 
 def _load_direct(lib: ctypes.CDLL):
-    path = _build.DIRECT_CALLS_PATH
-    if not path.exists():
-        raise RuntimeError(
-            f"{path.name} is not built (expected at {path}); build it with "
-            "`python -c 'import __graft_entry__ as g; g.build()'` from the repository root")
-    spec = importlib.util.spec_from_file_location("direct_calls", path)
-    module = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(module)
     if _raw_stream is None:
         return None
-    module.bind(_raw_stream, {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _SIGNATURES})
+    path = _build.DIRECT_CALLS_PATH
+    try:
+        spec = importlib.util.spec_from_file_location("direct_calls", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        built_for = module.torch_version, module.python_version
+        if built_for != (torch.__version__.split("+")[0], sys.hexversion >> 16):
+            raise ImportError("built for torch {}, Python {:#x}".format(*built_for))
+        module.bind(_raw_stream, {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _SIGNATURES})
+    except (ImportError, OSError, AttributeError, KeyError, ValueError) as e:
+        warnings.warn(f"{path.name} is not used, small calls take some microseconds more ({e}); build it with "
+                      "`python -c 'import __graft_entry__ as g; g.build()'` from the repository root",
+                      RuntimeWarning, stacklevel=3)
+        return None
     return module
 
 

@@ -6,6 +6,7 @@
 // by this host work: through Python checks and ctypes a norm took 7.6 us, context attention 14.5 us,
 // decode attention 16 us and RoPE with the append 21.9 us of host time.
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <initializer_list>
 
@@ -15,14 +16,16 @@ namespace {
 
 PyObject* g_raw_stream = nullptr;  // torch._C._cuda_getCurrentRawStream
 
+#define MAS_EACH_FN(F)                    \
+  F(mas_fused_add_rmsnorm_bf16)           \
+  F(mas_fused_add_rmsnorm_quant_fp8)      \
+  F(mas_silu_and_mul_bf16)                \
+  F(mas_silu_and_mul_quant_fp8)           \
+  F(mas_rope_append_paged_kv_cache_bf16)  \
+  F(mas_paged_decode_attention_bf16)      \
+  F(mas_paged_context_attention_bf16)
 #define MAS_FN(name) decltype(&name) g_##name = nullptr;
-MAS_FN(mas_fused_add_rmsnorm_bf16)
-MAS_FN(mas_fused_add_rmsnorm_quant_fp8)
-MAS_FN(mas_silu_and_mul_bf16)
-MAS_FN(mas_silu_and_mul_quant_fp8)
-MAS_FN(mas_rope_append_paged_kv_cache_bf16)
-MAS_FN(mas_paged_decode_attention_bf16)
-MAS_FN(mas_paged_context_attention_bf16)
+MAS_EACH_FN(MAS_FN)
 #undef MAS_FN
 
 using at::ScalarType;
@@ -348,28 +351,34 @@ PyObject* context_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
-// bind(raw_stream, {C entry point's name: its address}): called once, when the kernel library is loaded.
+// bind(raw_stream, {C entry point's name: its address}): called once, when the kernel library is loaded. Raises,
+// with what was bound before still in place, if a name is missing or the library's version is not that of the
+// header this file was compiled with, whose signatures it calls.
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 2 || !PyDict_Check(a[1])) {
     PyErr_SetString(PyExc_TypeError, "bind(raw_stream, addresses)");
     return nullptr;
   }
-  Py_INCREF(a[0]);
-  g_raw_stream = a[0];
-  const auto at_name = [&](const char* name, auto& fn) {
+  const auto at_name = [&](const char* name) {
     PyObject* v = PyDict_GetItemString(a[1], name);
     void* p = v ? PyLong_AsVoidPtr(v) : nullptr;
     if (p == nullptr && !PyErr_Occurred()) PyErr_Format(PyExc_KeyError, "%s", name);
-    fn = reinterpret_cast<std::decay_t<decltype(fn)>>(p);
-    return p != nullptr;
+    return p;
   };
-#define MAS_BIND(name) at_name(#name, g_##name)
-  if (!(MAS_BIND(mas_fused_add_rmsnorm_bf16) && MAS_BIND(mas_fused_add_rmsnorm_quant_fp8) &&
-        MAS_BIND(mas_silu_and_mul_bf16) && MAS_BIND(mas_silu_and_mul_quant_fp8) &&
-        MAS_BIND(mas_rope_append_paged_kv_cache_bf16) && MAS_BIND(mas_paged_decode_attention_bf16) &&
-        MAS_BIND(mas_paged_context_attention_bf16)))
+  void* const version = at_name("mas_version");
+#define MAS_FIND(name) void* const p_##name = PyErr_Occurred() ? nullptr : at_name(#name);
+  MAS_EACH_FN(MAS_FIND)
+#undef MAS_FIND
+  if (PyErr_Occurred()) return nullptr;
+  if (const int v = reinterpret_cast<decltype(&mas_version)>(version)(); v != MAS_VERSION) {
+    PyErr_Format(PyExc_ValueError, "compiled for version %d of the kernel library, loaded with %d", MAS_VERSION, v);
     return nullptr;
-#undef MAS_BIND
+  }
+#define MAS_SET(name) g_##name = reinterpret_cast<decltype(g_##name)>(p_##name);
+  MAS_EACH_FN(MAS_SET)
+#undef MAS_SET
+  Py_INCREF(a[0]);
+  Py_XSETREF(g_raw_stream, a[0]);
   Py_RETURN_NONE;
 }
 
@@ -387,4 +396,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "direct_calls", nullptr, -1, method
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_direct_calls() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit_direct_calls() {
+  PyObject* m = PyModule_Create(&module);
+  // what this file was compiled for: its caller binds it under the same torch and Python only
+  if (m != nullptr && (PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0 ||
+                       PyModule_AddIntConstant(m, "python_version", PY_VERSION_HEX >> 16) < 0))
+    Py_CLEAR(m);
+  return m;
+}

@@ -25,7 +25,7 @@ int device_cu_count(int* cus) {
 
 }  // namespace mas
 
-extern "C" int mas_version(void) { return (0 << 16) | (1 << 8) | 0; }
+extern "C" int mas_version(void) { return MAS_VERSION; }
 
 extern "C" const char* mas_status_string(int status) {
   switch (status) {

@@ -2,6 +2,8 @@
 form they take, and None, with nothing done, for every form they leave to the wrappers."""
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -32,6 +34,54 @@ def test_direct_calls_leave_other_forms_to_the_wrappers(mas):
         d.bind(None, {})
     d.bind(mas._lib._raw_stream, {n: mas._lib.ctypes.cast(getattr(mas._lib.load(), n), mas._lib.ctypes.c_void_p).value
                                   for n in mas._lib.exported_symbols()})
+
+
+def _addresses(mas):
+    lib = mas._lib.load()
+    return {n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in mas._lib.exported_symbols()}
+
+
+def test_the_library_loads_without_the_extension(mas, monkeypatch, tmp_path):
+    """No extension, one that is none, or one built for another torch: a warning, and the wrappers serve."""
+    lib = mas._lib.load()
+    other = tmp_path / "direct_calls.so"
+    other.write_text("not a library")
+    for path in (tmp_path / "absent.so", other):
+        monkeypatch.setattr(mas._lib._build, "DIRECT_CALLS_PATH", path)
+        with pytest.warns(RuntimeWarning, match="is not used"):
+            assert mas._lib._load_direct(lib) is None
+    monkeypatch.undo()
+    monkeypatch.setattr(torch, "__version__", "0.0.1+other")
+    with pytest.warns(RuntimeWarning, match="built for torch"):
+        assert mas._lib._load_direct(lib) is None
+    monkeypatch.undo()
+    assert mas._lib._load_direct(lib) is not None
+
+
+def test_the_extension_is_bound_to_its_own_library_version_only(mas):
+    mas.load_library()
+    other = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: 1 << 24)
+    with pytest.raises(ValueError, match="version"):
+        mas._lib.direct.bind(mas._lib._raw_stream,
+                             _addresses(mas) | {"mas_version": ctypes.cast(other, ctypes.c_void_p).value})
+
+
+def test_a_build_without_a_compiler_goes_on_without_the_extension(mas, monkeypatch, tmp_path):
+    monkeypatch.setattr(mas._lib._build, "DIRECT_CALLS_PATH", tmp_path / "direct_calls.so")
+    monkeypatch.setenv("CXX", str(tmp_path / "no-compiler"))
+    with pytest.warns(RuntimeWarning, match="failed"):
+        assert mas._lib._build.build_direct_calls() is None
+
+
+@pytest.mark.gpu
+def test_a_failed_bind_leaves_the_calls_bound(mas, dev):
+    mas.load_library()
+    d = mas._lib.direct
+    some = dict(list(_addresses(mas).items())[:3])
+    for names in ({}, some, _addresses(mas) | {"mas_silu_and_mul_bf16": None}):
+        with pytest.raises((KeyError, TypeError)):
+            d.bind(None, names)
+    assert d.silu_and_mul(torch.ones(2, 64, device=dev).bfloat16(), torch.empty(2, 32, device=dev).bfloat16()) == 0
 
 
 @pytest.mark.gpu
