@@ -173,7 +173,7 @@ def trtllm_batch_decode_with_kv_cache(query: torch.Tensor, kv_cache, workspace_b
                                              float(bmm1_scale), float(bmm2_scale), out, kv_layout, qs, qs_host,
                                              error_flags)
         return out
-    if _lib.direct is not None and (st := _lib.direct.decode_attention(
+    if workspace_buffer is not None and _lib.direct is not None and (st := _lib.direct.decode_attention(
             query, kv_cache, workspace_buffer, block_tables, seq_lens, bmm1_scale, bmm2_scale, out, kv_layout,
             error_flags, out_quant_scale)) is not None:
         if st:

@@ -3,6 +3,7 @@ form they take, and None, with nothing done, for every form they leave to the wr
 from __future__ import annotations
 
 import ctypes
+import timeit
 
 import pytest
 import torch
@@ -34,6 +35,17 @@ def test_direct_calls_leave_other_forms_to_the_wrappers(mas):
         d.bind(None, {})
     d.bind(mas._lib._raw_stream, {n: mas._lib.ctypes.cast(getattr(mas._lib.load(), n), mas._lib.ctypes.c_void_p).value
                                   for n in mas._lib.exported_symbols()})
+
+
+def test_a_form_left_to_the_wrappers_costs_little(mas):
+    """A refusal is a comparison and a return (0.1-0.2 us); as a C++ exception it took 3-4 us of the call."""
+    mas.load_library()
+    d, norm = mas._lib.direct, _norm_args()
+    for call in (lambda: d.fused_add_rmsnorm(*norm), lambda: d.silu_and_mul_quant(*norm[:2], 1.0),
+                 lambda: d.decode_attention(*[None] * 11), lambda: d.context_attention(*[None] * 14),
+                 lambda: d.rope_append(*norm, 64, *[None] * 10)):
+        assert call() is None
+        assert min(timeit.repeat(call, number=1000, repeat=20)) / 1000 < 1.5e-6
 
 
 def _addresses(mas):
