@@ -160,6 +160,8 @@ def test_attention_matches_the_general_way(mas, dev, layout, quant):
     q = qkv[:, : 8 * 64].view(11, 8, 64)
     a, b = out_of(q), out_of(q)
     for w in (ws, None):
+        a.view(torch.uint8).fill_(17)
+        b.view(torch.uint8).fill_(34)
         assert d.context_attention(q, kv, w, tables, lens, cu, 8, 40, 0.1, 1.0, a, layout, flags, quant) == 0
         mas.attention._context(q, kv, tables, lens, cu, 8, 0.1, 1.0, b, layout, flags, quant, w, 40)
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
@@ -202,3 +204,38 @@ def test_rope_append_matches_the_general_way(mas, dev, beta, layout, neox):
         mas.fused.apply_rope_and_append_paged_kv_cache(pos[:4], *args[1:], None, layout)
     with pytest.raises(ValueError, match="head_dim"):
         mas.fused.apply_rope_and_append_paged_kv_cache(pos, q, k, v, 32, *args[5:], None, layout)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["NHD", "HND"])
+@pytest.mark.parametrize("scaled", [False, True])
+def test_rope_append_takes_the_layers_forms(mas, dev, layout, scaled):
+    """The native call itself, of which the public one would hide a refusal."""
+    mas.load_library()
+    d = mas._lib.direct
+    kv, tables, _, _ = _attention(dev, layout)
+    pos = torch.tensor([0, 39, 3, 4, 16], dtype=torch.int32, device=dev)
+    batch = torch.tensor([0, 0, 1, 1, 1], dtype=torch.int32, device=dev)
+    indptr = torch.tensor([0, 3, 6], dtype=torch.int32, device=dev)
+    table = mas.rope.cos_sin_cache(64, 64, 1e6).to(dev)
+    flags = torch.zeros(1, dtype=torch.int32, device=dev)
+    scale = (mas.fused.llama_4_q_scale_table(0.1, 16, 4, dev), 16) if scaled else (None, 0)
+    qkv = torch.randn(5, 12 * 64, device=dev).bfloat16()
+    got = []
+    for native in (True, False):
+        x, cache = qkv.clone(), (kv[0].clone(), kv[1].clone())
+        q, k, v = x[:, :512], x[:, 512:640], x[:, 640:].unflatten(-1, (2, 64))
+        args = [pos, q, k, v, 64, table, True, batch, cache, tables.flatten(), indptr, layout, flags]
+        if native:
+            assert d.rope_append(*args, *scale) == 0
+        else:
+            mas.fused._fused(*args, *((0.1, 16) if scaled else ()))
+        got.append((x, *cache))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and int(flags.item()) == 0
+    assert not torch.equal(got[0][0], qkv) and not torch.equal(got[0][1], kv[0])
+    call, before = [*args, *scale], x.clone()
+    for at, other in ((0, pos[:4]), (0, pos.long()), (1, q[:, :500]), (1, q.float()), (2, k[:, :64]), (3, v[:4]), (4, 32),
+                      (5, table[:, :32]), (5, table.double()), (6, 1), (7, batch.cpu()), (8, list(cache)),
+                      (9, tables), (10, indptr.long()), (11, "DNH"), (12, flags.float()), (13, table[0])):
+        assert d.rope_append(*call[:at], other, *call[at + 1:]) is None
+    assert torch.equal(x, before)

@@ -3,10 +3,11 @@ halves and tiles, for every workgroup shape and page mode, with scores whose run
 move in a first half, a second half and not at all."""
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
-from conftest import bits
+from conftest import ATOL, RTOL, bits
 from oracle import ops
 from test_gpu_context_attention import SPLIT_WS, _case, _check, _run
 
@@ -16,7 +17,8 @@ LENGTHS = [(1, 1), (31, 31), (32, 32), (33, 33), (2, 34), (64, 64), (65, 65), (1
 
 
 @pytest.mark.parametrize("dim", [64, 128])
-@pytest.mark.parametrize("hq,hk", [(8, 2), (24, 2), (3, 1)])      # four and eight wavefronts, heads left over
+# four and eight wavefronts, one head per workgroup, and groups that leave wavefronts without a head
+@pytest.mark.parametrize("hq,hk", [(8, 2), (24, 2), (3, 1), (5, 1), (7, 1), (9, 1), (11, 1)])
 @pytest.mark.parametrize("page_size", [4, 8, 16, 32, 64])
 def test_half_step_edges(mas, dev, dim, hq, hk, page_size):
     q_lens, kv_lens = [n for n, _ in LENGTHS], [n for _, n in LENGTHS]
@@ -28,7 +30,7 @@ def test_half_step_edges(mas, dev, dim, hq, hk, page_size):
             factor = 24.0 if r % 3 == 1 and p >= 32 else (6.0 if r % 3 == 2 and p >= 64 else 1.0)
             kc[int(tables[r, p // page_size]), p % page_size] *= factor
     want = ops.paged_context_attention(bits(q), bits(kc), bits(vc), tables.numpy(), seq.numpy(), cu.numpy(), 0.1)
-    for ws_bytes in (16, SPLIT_WS):
+    for ws_bytes in (16, SPLIT_WS):  # rows this short are not split, whatever the workspace holds
         got = _run(mas, dev, q, kc, vc, tables, seq, cu, 0.1, ws_bytes=ws_bytes, max_kv=max(kv_lens))
         _check(bits(got), want, min_exact=0.5)
 
@@ -112,3 +114,38 @@ def test_split_ranges_end_at_every_half(mas, dev, dim, hq, hk, page_size):
     assert not torch.all(ws == 255)
     want = ops.paged_context_attention(bits(q), bits(kc), bits(vc), tables.numpy(), seq.numpy(), cu.numpy(), dim ** -0.5)
     _check(bits(got), want, min_exact=0.5)
+
+
+def _softmax64(q, kc, vc, table, kv_len, scale):
+    """float64 causal attention of the last len(q) of kv_len positions, one kv head: IEEE's NaN and infinities."""
+    rows = [c[table.long()].flatten(0, 1)[:kv_len, 0].double() for c in (kc, vc)]
+    scores = torch.einsum("thd,pd->htp", q.double(), rows[0]) * scale
+    at = torch.arange(kv_len)[None, :] > torch.arange(kv_len - len(q), kv_len)[:, None]
+    p = torch.softmax(scores.masked_fill(at, -float("inf")), -1)
+    return torch.stack([torch.stack([(row[:n, None] * rows[1][:n]).sum(0) for row, n in zip(
+        head, range(kv_len - len(q) + 1, kv_len + 1))]) for head in p]).transpose(0, 1)
+
+
+SPECIALS = ["inf key", "nan key", "inf value", "nan value"]
+
+
+@pytest.mark.parametrize("what,kv_len,ws_bytes", [("nan query", 200, 16), *((w, 200, 16) for w in SPECIALS),
+                                                  *((w, 1500, SPLIT_WS) for w in SPECIALS)])
+@pytest.mark.parametrize("at", [3, 40, 70, 170])  # a first and a second half of the first tile and of later ones
+@pytest.mark.parametrize("page_size,hq", [(4, 4), (16, 4), (64, 12)])
+def test_nan_and_infinity(mas, dev, what, at, kv_len, ws_bytes, page_size, hq):
+    """A query that is not a number gets NaN and no other token does; a key's infinite element makes scores
+    of +inf (NaN outputs) and -inf (weight 0) by the query's sign; values pass into their column alone."""
+    n, dim = 20, 64
+    q, kc, vc, tables, seq, cu = _case(at, [n], [kv_len], hq, 1, dim, page_size)
+    where, special = (int(tables[0, at // page_size]), at % page_size, 0), float(what[:3])
+    if what == "nan query":
+        q[7, 1, 5] = special
+    else:
+        (kc if "key" in what else vc)[where][5] = special
+    want = _softmax64(q, kc, vc, tables[0], kv_len, 0.125)
+    got = _run(mas, dev, q, kc, vc, tables, seq, cu, 0.125, ws_bytes=ws_bytes, max_kv=kv_len).double().cpu()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    finite = want.isfinite()
+    assert finite.any() == (what != "nan key")
+    np.testing.assert_allclose(got[finite], want[finite], rtol=RTOL, atol=ATOL)
