@@ -873,12 +873,13 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   // masked score), which the test catches as well. The split partials carry this m with their sums. A lane adds
   // its 32 p of a tile in one chain, t_run over its first half, and each tile's sum to l_run; the two
   // lanes of a row add theirs after the last tile.
-  auto move_reference = [&](const f32x16& s, bool second, bool over, bf16x8 (&pbo)[2]) {
+  auto move_reference = [&](const f32x16& s, bool second, uint64_t over, bf16x8 (&pbo)[2]) {
     float mh = kNegInf;
 #pragma unroll
     for (int j = 0; j < 16; ++j) mh = fmaxf(mh, s[j]);
     const float mx = fmaxf(mh, __shfl_xor(mh, 32));  // the same in both lanes of a row, either of which moves it
-    const bool moves = (__shfl_xor(over ? 1 : 0, 32) | (over ? 1 : 0)) != 0;
+    asm volatile("" : "+s"(over));  // keeps what follows in this seldom taken branch
+    const bool moves = __builtin_amdgcn_inverse_ballot_w64(over | over >> 32 | over << 32);
     const float m_new = moves ? fmaxf(m_run, mx) : m_run;
     // rows that had no finite score have O = 0 and l = 0: their factor is 1, as that of a row that stays is
     // (m c - m c rounded is not 0)
@@ -895,8 +896,8 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   // The weights of a tile's first or second half against the row's m, which moves where it must.
   auto weigh_half = [&](const f32x16& s, bool second, bf16x8 (&pbo)[2]) {
     float sum = weigh(s, m_run * c, second ? t_run : 0.f, pbo);
-    const bool over = !(sum <= kSumMost);
-    if (__builtin_amdgcn_ballot_w64(over) != 0) sum = move_reference(s, second, over, pbo);  // wavefront-uniform
+    const uint64_t over = __builtin_amdgcn_ballot_w64(!(sum <= kSumMost));  // the lanes, a wavefront-uniform mask
+    if (over != 0) sum = move_reference(s, second, over, pbo);
     if (second) l_run += sum;
     else t_run = sum;
   };
