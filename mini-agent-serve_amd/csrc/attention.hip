@@ -134,10 +134,15 @@ __device__ __forceinline__ u32x4 attn_load_v(const uint16_t* p) { return load_st
 // Wavefronts per workgroup of the split kernel: two in large grids with an even kv head count, the
 // neighbouring kv heads of one split, else one (head_dim 256: one, for LDS). A pair reads 512 adjacent bytes of each
 // position from one CU: 64 rows of up to 8192 positions, 24B heads, 212 -> 201 us, 123B heads 226 -> 214
-// us, 28 rows 109 -> 106 us, 24 rows of up to 3000 (123B) 41.8 -> 39.7 us. A pair also holds its slots until
-// both end: with fewer than kPairItems (row, kv head, split) work items, one or two rounds of the GPU's wavefront
-// slots, that costs more (4 rows of up to 20000, 2528 items: 38.8 -> 40.0 us; four heads per workgroup:
-// 203 us, 216 us, 107 us). LDS traffic is ordered within the wavefront only.
+// us, 28 rows 109 -> 106 us. A pair also holds its slots until both end, which costs where the GPU's 2048
+// wavefront slots (two per SIMD) are filled once or twice: the line lies at two rounds of (row, kv head,
+// split) items under the table's reach. Below it one head is better in most shapes (pairs, one: 4 rows of up to
+// 20000, 1280 items, 47.2, 46.1 us; 8 rows of 4 heads, 1280: 53.1, 45.9; 12 rows, 3840: 91.5, 89.7; but 64 rows of 4
+// heads of up to 1000, 2048: 23.0, 26.4), above it pairs (20 rows of up to 20000, 6400: 167.2, 170.5; 123B heads,
+// 32 rows of up to 8192, 8192: 98.5, 99.9); up to two rounds further it turns on the rows' own lengths, by up
+// to 7% (20 rows of up to 3000, 5120: 35.5, 36.5; 24 of up to 8192, 6144: 67.5, 65.8; 64 of up to 1000, 4096: 36.4,
+// 34.3 us). Four heads per workgroup: 203 us, 216 us, 107 us for the first three. LDS traffic is ordered within
+// the wavefront only.
 constexpr int64_t kPairItems = 4096;
 // Wavefronts per SIMD the split kernel's registers are capped for (two load buffers of a step each).
 constexpr int kAttnMinWaves = 2;

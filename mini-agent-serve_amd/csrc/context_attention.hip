@@ -17,7 +17,8 @@
 // key / value tile they stage in LDS serves 128 (256) query rows. Per tile:
 //   S^T = K Q^T on MFMA (v_mfma_f32_32x32x16_bf16; A = 32 key rows read from LDS, B = the
 //   wavefront's 32 query rows, held in registers), causal mask, online softmax per query row (its
-//   running max moved only by rises of more than 2^8 in p, so O is seldom rescaled), then
+//   reference moved only where a lane's weights of the tile sum to more than 2^8, so O is seldom
+//   rescaled), then
 //   O^T += V^T P^T on MFMA, where P^T is packed to bf16 straight from the S^T accumulators and V^T
 //   is read from the row-major value tile with gfx950's transposing LDS read (ds_read_b64_tr_b16:
 //   in each group of 16 lanes, lane 4a + b receives element b of the 4-element rows that lanes
@@ -28,13 +29,17 @@
 // Keys and values have two LDS buffers each. With pages of at least 8 slots the tiles go to LDS by DMA,
 // issued among the MFMAs, keys a tile ahead of values (tile i + 2's keys and tile i + 1's values in
 // flight), one barrier per tile; smaller pages stage a tile through registers, two barriers per tile.
-// What bounds it: the card's power (the clock settles near 2 GHz under this load, and falls as the loop
-// gets denser), the 32 MFMAs per tile and wavefront (2048 of about 3200 cycles per tile for a SIMD's two
-// wavefronts), and the latency of the tiles' loads. Before the halves, the unpadded LDS rows (32 DMA
-// instructions per tile for 35 or 40, no bank conflicts) and the DMA among the MFMAs, a tile's scores
-// ran beside the whole previous tile's softmax, which waited for its maximum: 4 x 4096 tokens of 96 heads
-// over 8 took 1656 us, then 1571 (1050 TFLOP/s; a large bf16 matrix product reaches 1537 on this card);
-// 4 x 2048 of 32 heads 158 -> 150 us, 6 ragged prompts after cached ones 206 -> 191 us.
+// What bounds it: the card's power (the clock settles near 1.95 GHz under this load, and falls as the loop
+// gets denser), the 32 MFMAs per tile and wavefront (2048 of about 3300 cycles per tile for a SIMD's two
+// wavefronts; over a whole call the matrix pipe is busy 47% of the cycles at 4 x 2048 tokens of 32 heads
+// over 8, 53% at 4 x 4096 of 96), and the latency of the tiles' loads. Before the halves, the unpadded LDS
+// rows (32 DMA instructions per tile for 35 or 40, 1-3% of the LDS cycles lost to bank conflicts for 33%),
+// the DMA among the MFMAs, the pages found a tile ahead and the outputs through LDS, a tile's scores ran
+// beside the whole previous tile's softmax, which waited for its maximum. All of them together: 4 x 4096
+// 1733 -> 1596 us (1034 TFLOP/s; a large bf16 matrix product reaches 1537 on this card), 4 x 2048
+// 165.6 -> 151.3 us, 6 ragged prompts after cached ones 216 -> 200 us. (Every "a -> b us" here compares both
+// sides on one card in one session; cards and sessions differ by up to 8%, so figures of different pairs
+// do not follow each other.)
 #include <algorithm>
 
 #include "device.h"
@@ -152,16 +157,16 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, lds_u16* dst, in
 constexpr int kWaitVmcnt0 = 0x0f70;
 
 // How a tile's key / value rows find their pages (the block-table reads of a tile):
-//   kPagesTile  - pages of at least a tile: the tile lies in one page, one scalar read per tile;
+//   kPagesTile  - pages of at least a tile: the tile lies in one page (LDS DMA);
 //   kPagesMulti8 / 16 / 32 - pages of 8, 16 or 32 slots (LDS DMA, as kPagesTile): the tile's pages
 //                 are dealt out to the wavefronts, each page loaded under a buffer resource of its own;
 //   kPagesLane  - pages of 1-4 slots, and layouts whose in-page byte offsets do not fit the DMA
 //                 modes' 31 bits: each lane reads the page of each of its rows (vector loads) into
 //                 registers, staged into LDS a tile ahead (two barriers per tile).
-// Vector loads of block-table entries make the compiler wait for them, and such waits cover every
-// vector load issued before them, the next tiles' key / value loads included: the DMA modes read
-// them as scalars. (Modes for pages of at least a thread-row step, staged through registers with
-// scalar page reads, served pages of 8-32 slots before the DMA modes.)
+// A vector load of a block-table entry makes the compiler wait for it where it is used, and such a wait
+// covers every vector load issued before it, the next tiles' key / value loads included: the DMA modes
+// load 64 entries at once, a tile before the first of them is used, so that the tiles' own wait covers
+// them too (the first two tiles' entries are scalar loads).
 constexpr int kPagesLane = 0, kPagesTile = 2;
 // kPagesMulti8 + i: pages of 8 << i slots (i < 3)
 constexpr int kPagesMulti8 = 4, kPagesMulti16 = 5, kPagesMulti32 = 6;
@@ -927,8 +932,9 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void context_attn(ContextA
   };
 
   TileRegs tr;
-  // Software pipeline over tiles: tile it + 1's scores (MFMA, keys from the other LDS buffer) are
-  // computed in the same block as tile it's softmax (VALU), so the two overlap; then tile it's P.V.
+  // Software pipeline over tiles: step it takes tile it's second half through its weights and both halves
+  // through P.V, and tile it + 1 (keys from the other LDS buffer) through its scores and its first half's
+  // weights; the prologue does the latter for the first tile, last_step the former for the last.
   // Buffer (it - it_begin) & 1 holds tile it, the other one tile it + 1 (staged after the barrier
   // that ends every read of tile it - 1, which used that buffer). The parity is counted from the
   // workgroup's first tile, so that it is a constant at each call of step even where the first tile
